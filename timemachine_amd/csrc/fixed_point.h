@@ -80,6 +80,43 @@ TM_HD inline void round_to_fixed3(double a, double b, double c, uint64_t &fa, ui
     fc = round_to_fixed(c);
 }
 
+// round(a * b) to fixed point with one rounding: the add-magic step is a fused
+// multiply-add, so the product is never rounded by itself (one instruction
+// less a component than multiply, then add). Products of 2^51 and more take
+// the rounded product's general path.
+TM_HD inline uint64_t product_to_fixed(double a, double b) {
+    const double p = a * b;
+    if (__builtin_fabs(p) < 0x1p51) {
+        const double t = __builtin_fma(a, b, 0x1.8p52);
+        uint64_t bits;
+        __builtin_memcpy(&bits, &t, sizeof(bits));
+        return bits - FIXED_MAGIC_BITS;
+    }
+    return round_to_fixed(p);
+}
+
+// product_to_fixed(s, v) of three components |v| <= vmax, with one range test
+// for the common case: small = 2^51 / vmax rounded down (fixed_small_factor).
+TM_HD inline double fixed_small_factor(double vmax) { return 0x1.fffffffffff00p50 / vmax; }
+TM_HD inline void product3_to_fixed(double s, double small, double x, double y, double z, uint64_t &fx, uint64_t &fy,
+                                    uint64_t &fz) {
+    if (__builtin_fabs(s) < small) { // false for NaN
+        const double tx = __builtin_fma(s, x, 0x1.8p52), ty = __builtin_fma(s, y, 0x1.8p52),
+                     tz = __builtin_fma(s, z, 0x1.8p52);
+        uint64_t bx, by, bz;
+        __builtin_memcpy(&bx, &tx, sizeof(bx));
+        __builtin_memcpy(&by, &ty, sizeof(by));
+        __builtin_memcpy(&bz, &tz, sizeof(bz));
+        fx = bx - FIXED_MAGIC_BITS;
+        fy = by - FIXED_MAGIC_BITS;
+        fz = bz - FIXED_MAGIC_BITS;
+        return;
+    }
+    fx = product_to_fixed(s, x);
+    fy = product_to_fixed(s, y);
+    fz = product_to_fixed(s, z);
+}
+
 // f32 value -> fixed point with scale 2^k (scale must be a power of two).
 TM_HD inline uint64_t f32_to_fixed(float v, float scale) {
     return round_to_fixed(static_cast<double>(v * scale));

@@ -257,12 +257,12 @@ __global__ __launch_bounds__(256) void k_pair_list_hvp(const PairListArgs a, con
         const double dwdl = (ofi - ofj) * cutoff;
         const Dual dw((pli + ofi * lam) * cutoff - (plj + ofj * lam) * cutoff, dwdl * vl);
         const double *box = a.boxes + s * 9;
-        const double L[3] = {box[0], box[4], box[8]};
+        const BoxAxis axis[3] = {BoxAxis(box[0]), BoxAxis(box[4]), BoxAxis(box[8])};
         Dual dv[3];
         for (int d = 0; d < 3; d++) {
             // the image shift is a constant: the tangent is vx_i - vx_j
             const double tan = v.vx ? v.vx[gi * 3 + d] - v.vx[gj * 3 + d] : 0.0;
-            dv[d] = Dual(min_image_d(a.x[gi * 3 + d] - a.x[gj * 3 + d], L[d], 1.0 / L[d]), tan);
+            dv[d] = Dual(axis[d].delta(a.x[gi * 3 + d], a.x[gj * 3 + d]), tan);
         }
         const double d2 = __builtin_fma(dw.v, dw.v, pair_d2(dv[0].v, dv[1].v, dv[2].v));
         in = d2 < cutoff * cutoff;
@@ -349,8 +349,9 @@ __global__ __launch_bounds__(64) void k_tiles_hvp(
             continue;
         }
         const NbSys Sd = sys[s];
-        const double bx = boxes[s * 9 + 0], by = boxes[s * 9 + 4], bz = boxes[s * 9 + 8];
-        const double ibx = 1.0 / bx, iby = 1.0 / by, ibz = 1.0 / bz;
+        const BoxAxis gx(boxes[s * 9 + 0]), gy(boxes[s * 9 + 4]), gz(boxes[s * 9 + 8]);
+        const double bx = gx.edge, by = gy.edge, bz = gz.edge;
+        const double ibx = gx.inv, iby = gy.inv, ibz = gz.inv;
         const double beta = static_cast<double>(Sd.beta);
         const double cut2 = Sd.cutoff_d * Sd.cutoff_d;
         const double vl = v.vls ? v.vls[s] : v.vl;

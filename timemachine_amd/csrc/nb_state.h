@@ -50,6 +50,14 @@ constexpr int NB_STATUS_BOX_TOO_SMALL = 1;
 constexpr int NB_STATUS_BOX_NOT_ORTHO = 2;
 constexpr int NB_STATUS_TILE_OVERFLOW = 4;
 
+// Partial sums of u ([0]) and du/dl ([1]) of one system, and the waves that have
+// added to them in this launch. All zero between launches.
+constexpr int NB_RED_SLOTS = 32;
+struct alignas(128) NbRedSlot {
+    uint64_t v[2];
+    uint32_t waves;
+};
+
 struct NbSys {
     int atom0;    // first global atom (rows of x / du_dx / params)
     int n_atoms;  // atoms of the system
@@ -142,6 +150,10 @@ struct NbState {
     // [total_blocks * NB_MAX_PIECES] (empty for views: one piece)
     DeviceArray<uint32_t> piece_buf;
     DeviceArray<int> piece_cnt;
+    // [6 * total_slots] the tiles' sums of force and parameter derivatives by slot,
+    // zero between launches (empty for views: tiles add to the atoms)
+    DeviceArray<uint64_t> sorted_acc;
+    DeviceArray<NbRedSlot> red_slots; // [S * NB_RED_SLOTS] (empty for views: u and du_dl are added directly)
     DeviceArray<double> nblist_x; // [sum n_atoms * 3] coordinates at the last build
     DeviceArray<double> nblist_box; // [S * 9]
 
@@ -201,6 +213,8 @@ struct NbState {
         uint64_t *u,
         hipStream_t stream,
         int grid_override = 0) const;
+
+    void add_sorted(uint64_t *du_dx, uint64_t *du_dp, hipStream_t stream) const; // sorted_acc to the outputs
 
     // d(du/dlambda)/dp [*, 3] (rows atom0 + i), accumulated with the du_dp
     // fixed-point exponents. Uses the tiles and sorted data of the last

@@ -338,10 +338,12 @@ __global__ __launch_bounds__(SORT_THREADS) void k_sort(
 // grid (ceil(max_slots / 256), S): sorted FP32 coordinates and parameters.
 // w = (plane + offset * lambda) * cutoff and dw/dlambda = offset * cutoff, in
 // f64 before rounding to FP32 (kernels/k_lambda_transformer_jit.cuh:25-55 with
-// the identity transform).
+// the identity transform). With boxes the coordinates are wrapped onto the box's
+// grid (BoxAxis), as the pair kernels expect them; without, they are copied.
 __global__ void k_gather(
     const NbSys *__restrict__ sys,
     const double *__restrict__ x,
+    const double *__restrict__ boxes,
     const double *__restrict__ params,
     const double *__restrict__ params1,
     const int *__restrict__ plane,
@@ -373,7 +375,13 @@ __global__ void k_gather(
     const int of = offset ? offset[g] : 0;
     const double w = (pl + of * lam) * S.cutoff_d;
     const double dw_dl = of * S.cutoff_d;
-    pos[S.slot0 + slot] = make_double4(x[g * 3 + 0], x[g * 3 + 1], x[g * 3 + 2], w);
+    double4 p4 = make_double4(x[g * 3 + 0], x[g * 3 + 1], x[g * 3 + 2], w);
+    if (boxes) {
+        p4.x = BoxAxis(boxes[s * 9 + 0]).wrap(p4.x);
+        p4.y = BoxAxis(boxes[s * 9 + 4]).wrap(p4.y);
+        p4.z = BoxAxis(boxes[s * 9 + 8]).wrap(p4.z);
+    }
+    pos[S.slot0 + slot] = p4;
     if (params) {
         if (S.interp && params1) {
             // parameter interpolation with the identity transform
@@ -1105,11 +1113,15 @@ void NbState::init(const std::vector<NbSys> &sys_in, const std::vector<int> &sub
     bb_ext.alloc(total_blocks);
     piece_buf.alloc(static_cast<size_t>(total_blocks) * NB_MAX_PIECES * TILE);
     piece_cnt.alloc(static_cast<size_t>(total_blocks) * NB_MAX_PIECES);
+    sorted_acc.alloc(static_cast<size_t>(total_slots) * 6);
+    red_slots.alloc(static_cast<size_t>(S) * NB_RED_SLOTS);
     nblist_x.alloc(static_cast<size_t>(total_atoms_end) * 3);
     nblist_box.alloc(static_cast<size_t>(S) * 9);
     status.zero();
     tile_count.zero();
     tile_prefix.zero();
+    sorted_acc.zero();
+    red_slots.zero();
     nblist_x.zero();
     nblist_box.zero();
     launch_fill_i32(rebuild.ptr, S, 1, 0);
@@ -1178,7 +1190,7 @@ void NbState::build_only(const double *x, const double *boxes, hipStream_t strea
                                           nblist_box.ptr, tile_count.ptr);
     TM_LAUNCH_CHECK();
     k_gather<<<dim3(ceil_div(max_slots, 256), S), 256, 0, stream>>>(sys.ptr, x, nullptr, nullptr, nullptr, nullptr,
-                                                                    nullptr, 0.0, perm.ptr, pos.ptr, par.ptr, nullptr);
+                                                                    nullptr, nullptr, 0.0, perm.ptr, pos.ptr, par.ptr, nullptr);
     TM_LAUNCH_CHECK();
     k_block_bounds<<<dim3(ceil_div(max_blocks, 4), S), 256, 0, stream>>>(sys.ptr, boxes, rebuild.ptr, pos.ptr,
                                                                          bb_ctr.ptr, bb_ext.ptr);
@@ -1216,7 +1228,7 @@ void NbState::prepare(
                                           nblist_box.ptr, tile_count.ptr);
     TM_LAUNCH_CHECK();
     k_gather<<<dim3(ceil_div(max_slots, 256), S), 256, 0, stream>>>(
-        sys.ptr, x, params, params1, plane, offset, lambdas, lambda0, perm.ptr, pos.ptr, par.ptr,
+        sys.ptr, x, boxes, params, params1, plane, offset, lambdas, lambda0, perm.ptr, pos.ptr, par.ptr,
         any_interp ? dpar.ptr : nullptr);
     TM_LAUNCH_CHECK();
     k_block_bounds<<<dim3(ceil_div(max_blocks, 4), S), 256, 0, stream>>>(sys.ptr, boxes, rebuild.ptr, pos.ptr,
