@@ -37,15 +37,33 @@ struct BondedIncidence {
 void build_bonded_incidence(int A, const std::vector<const std::vector<int> *> &idx, std::vector<int> &off,
                             std::vector<uint32_t> &items, std::vector<int> &slot0);
 
-// One thread per atom sums its slots and adds them to du_dx with a plain
-// read-modify-write (no other kernel writes du_dx meanwhile). The fixed-point
-// values are those the atomics would add, so the sums are bitwise the same.
-void launch_bonded_gather(const BondedIncidence &inc, const uint64_t *slots, uint64_t *du_dx, hipStream_t stream);
+// The pair tiles' force sums in sorted order: component c of global atom a is
+// sorted[c * slots + slot_of[a]], no sums for slot_of[a] < 0 or a >= atoms.
+struct SortedForces {
+    uint64_t *sorted;
+    size_t slots;
+    const int *slot_of;
+    int atoms; // 0: no sums
+};
+
+// du_dx[a] = its slots' sum + its sorted sums (cleared after the read). Nothing
+// else may write du_dx or the sums meanwhile. The fixed-point values are those
+// the atomics would add, so the sums are bitwise the same. inc.off may be null.
+void launch_atom_forces(const BondedIncidence &inc, const uint64_t *slots, const SortedForces &s0,
+                        const SortedForces &s1, uint64_t *du_dx, hipStream_t stream);
+
+// All bonded terms of a batch in one launch. With slots the per-atom forces go
+// to force slots (see above) instead of du_dx.
+struct BondedSet {
+    BondedTerms t[3];   // by BondedKind
+    uint64_t *slots[3]; // or nullptr
+};
+void launch_bonded_all(const BondedSet &b, const double *x, const double *lambdas, const int *red_idx, uint64_t *du_dx,
+                       uint64_t *du_dl, uint64_t *u, hipStream_t stream);
 
 // dl_dp: write d(du/dlambda)/dp into du_dp (every other output must be null).
-// slots: write the per-atom forces into force slots (see above) instead of du_dx.
 void launch_bonded(BondedKind kind, const BondedTerms &t, const double *x, const double *lambdas, double lambda0,
                    const int *red_idx, uint64_t *du_dx, uint64_t *du_dp, uint64_t *du_dl, uint64_t *u,
-                   hipStream_t stream, bool dl_dp = false, uint64_t *slots = nullptr);
+                   hipStream_t stream, bool dl_dp = false);
 
 } // namespace tmamd

@@ -27,11 +27,11 @@ __device__ __forceinline__ void term_context(const BondedTerms &t, int term, con
     red = red_idx ? red_idx[s] : 0;
 }
 
-__global__ void k_harmonic_bond(const BondedTerms t, const double *__restrict__ x, const double *__restrict__ lambdas,
-                                double lambda0, const int *__restrict__ red_idx, uint64_t *__restrict__ du_dx,
-                                uint64_t *__restrict__ du_dp, uint64_t *__restrict__ du_dl, uint64_t *__restrict__ u, int dl_dp,
-                                uint64_t *__restrict__ slots) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void harmonic_bond(const BondedTerms &t, const int b, const double *__restrict__ x,
+                                   const double *__restrict__ lambdas, double lambda0,
+                                   const int *__restrict__ red_idx, uint64_t *__restrict__ du_dx,
+                                   uint64_t *__restrict__ du_dp, uint64_t *__restrict__ du_dl,
+                                   uint64_t *__restrict__ u, int dl_dp, uint64_t *__restrict__ slots) {
     const bool active = b < t.n;
     double lam = 0.0;
     int red = -1;
@@ -72,11 +72,11 @@ __global__ void k_harmonic_bond(const BondedTerms t, const double *__restrict__ 
     }
 }
 
-__global__ void k_harmonic_angle(const BondedTerms t, const double *__restrict__ x, const double *__restrict__ lambdas,
-                                 double lambda0, const int *__restrict__ red_idx, uint64_t *__restrict__ du_dx,
-                                 uint64_t *__restrict__ du_dp, uint64_t *__restrict__ du_dl,
-                                 uint64_t *__restrict__ u, int dl_dp, uint64_t *__restrict__ slots) {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void harmonic_angle(const BondedTerms &t, const int a, const double *__restrict__ x,
+                                   const double *__restrict__ lambdas, double lambda0,
+                                   const int *__restrict__ red_idx, uint64_t *__restrict__ du_dx,
+                                   uint64_t *__restrict__ du_dp, uint64_t *__restrict__ du_dl,
+                                   uint64_t *__restrict__ u, int dl_dp, uint64_t *__restrict__ slots) {
     const bool active = a < t.n;
     double lam = 0.0;
     int red = -1;
@@ -120,12 +120,11 @@ __global__ void k_harmonic_angle(const BondedTerms t, const double *__restrict__
     }
 }
 
-__global__ void k_periodic_torsion(const BondedTerms t, const double *__restrict__ x,
-                                   const double *__restrict__ lambdas, double lambda0, const int *__restrict__ red_idx,
-                                   uint64_t *__restrict__ du_dx, uint64_t *__restrict__ du_dp,
-                                   uint64_t *__restrict__ du_dl, uint64_t *__restrict__ u, int dl_dp,
-                                   uint64_t *__restrict__ slots) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void periodic_torsion(const BondedTerms &t, const int q, const double *__restrict__ x,
+                                   const double *__restrict__ lambdas, double lambda0,
+                                   const int *__restrict__ red_idx, uint64_t *__restrict__ du_dx,
+                                   uint64_t *__restrict__ du_dp, uint64_t *__restrict__ du_dl,
+                                   uint64_t *__restrict__ u, int dl_dp, uint64_t *__restrict__ slots) {
     const bool active = q < t.n;
     double lam = 0.0;
     int red = -1;
@@ -173,29 +172,99 @@ __global__ void k_periodic_torsion(const BondedTerms t, const double *__restrict
     }
 }
 
-// Sum of the fixed-point force slots incident to each atom, added to du_dx
-// with a plain read-modify-write (one thread per atom owns its three words).
-__global__ void k_bonded_gather(const BondedIncidence inc, const uint64_t *__restrict__ slots,
-                                uint64_t *__restrict__ du_dx) {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= inc.A) {
-        return;
+template <BondedKind KIND>
+__device__ __forceinline__ void bonded_term(const BondedTerms &t, const int term, const double *x,
+                                            const double *lambdas, double lambda0, const int *red_idx, uint64_t *du_dx,
+                                            uint64_t *du_dp, uint64_t *du_dl, uint64_t *u, int dl_dp, uint64_t *slots) {
+    if constexpr (KIND == BondedKind::Bond) {
+        harmonic_bond(t, term, x, lambdas, lambda0, red_idx, du_dx, du_dp, du_dl, u, dl_dp, slots);
+    } else if constexpr (KIND == BondedKind::Angle) {
+        harmonic_angle(t, term, x, lambdas, lambda0, red_idx, du_dx, du_dp, du_dl, u, dl_dp, slots);
+    } else {
+        periodic_torsion(t, term, x, lambdas, lambda0, red_idx, du_dx, du_dp, du_dl, u, dl_dp, slots);
     }
-    const int e0 = inc.off[a], e1 = inc.off[a + 1];
-    if (e0 == e1) {
+}
+
+constexpr int TERM_BLOCK = 128;
+
+template <BondedKind KIND>
+__global__ __launch_bounds__(TERM_BLOCK) void k_bonded(const BondedTerms t, const double *__restrict__ x,
+                                                       const double *__restrict__ lambdas, double lambda0,
+                                                       const int *__restrict__ red_idx, uint64_t *__restrict__ du_dx,
+                                                       uint64_t *__restrict__ du_dp, uint64_t *__restrict__ du_dl,
+                                                       uint64_t *__restrict__ u, int dl_dp,
+                                                       uint64_t *__restrict__ slots) {
+    bonded_term<KIND>(t, blockIdx.x * TERM_BLOCK + threadIdx.x, x, lambdas, lambda0, red_idx, du_dx, du_dp, du_dl, u,
+                      dl_dp, slots);
+}
+
+// All three kinds in one launch: workgroups [0, g1) take bonds, [g1, g2) angles
+// and the rest torsions. What bounds a single system is the launch itself (4.5 us
+// a graph node for ~1 us of work on 6k atoms), so one instead of three.
+__global__ __launch_bounds__(TERM_BLOCK) void k_bonded_all(const BondedSet b, const int g1, const int g2,
+                                                           const double *__restrict__ x,
+                                                           const double *__restrict__ lambdas,
+                                                           const int *__restrict__ red_idx,
+                                                           uint64_t *__restrict__ du_dx, uint64_t *__restrict__ du_dl,
+                                                           uint64_t *__restrict__ u) {
+    const int g = blockIdx.x;
+    if (g < g1) {
+        bonded_term<BondedKind::Bond>(b.t[0], g * TERM_BLOCK + threadIdx.x, x, lambdas, 0.0, red_idx, du_dx, nullptr,
+                                      du_dl, u, 0, b.slots[0]);
+    } else if (g < g2) {
+        bonded_term<BondedKind::Angle>(b.t[1], (g - g1) * TERM_BLOCK + threadIdx.x, x, lambdas, 0.0, red_idx, du_dx,
+                                       nullptr, du_dl, u, 0, b.slots[1]);
+    } else {
+        bonded_term<BondedKind::Torsion>(b.t[2], (g - g2) * TERM_BLOCK + threadIdx.x, x, lambdas, 0.0, red_idx, du_dx,
+                                         nullptr, du_dl, u, 0, b.slots[2]);
+    }
+}
+
+// Force of every atom: the fixed-point slots of its terms plus the tiles' sums in
+// sorted order, which are cleared for the next launch. GATHER_LANES lanes share an
+// atom: one thread an atom walked the longest list alone (a ligand atom of ~60
+// slots, two dependent loads each: 17.8 us for one system of 6k atoms) and
+// wrote its three words by itself.
+constexpr int GATHER_LANES = 4;
+
+__global__ __launch_bounds__(256) void k_atom_forces(const BondedIncidence inc, const uint64_t *__restrict__ slots,
+                                                     const SortedForces s0, const SortedForces s1,
+                                                     uint64_t *__restrict__ du_dx) {
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    const int a = t / GATHER_LANES;
+    const int q = t % GATHER_LANES;
+    if (a >= inc.A) { // whole groups leave
         return;
     }
     uint64_t acc[3] = {0, 0, 0};
-    for (int e = e0; e < e1; e++) {
-        const uint64_t *g = slots + static_cast<size_t>(inc.items[e]) * 3;
-        acc[0] += g[0];
-        acc[1] += g[1];
-        acc[2] += g[2];
-    }
-    for (int d = 0; d < 3; d++) {
-        if (acc[d] != 0) {
-            du_dx[a * 3 + d] += acc[d];
+    if (inc.off) {
+        const int e1 = inc.off[a + 1];
+#pragma unroll 2
+        for (int e = inc.off[a] + q; e < e1; e += GATHER_LANES) {
+            const uint64_t *g = slots + static_cast<size_t>(inc.items[e]) * 3;
+            acc[0] += g[0];
+            acc[1] += g[1];
+            acc[2] += g[2];
         }
+    }
+    for (int m = 1; m < GATHER_LANES; m <<= 1) {
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            acc[d] += __shfl_xor(static_cast<unsigned long long>(acc[d]), m, 64);
+        }
+    }
+    if (q < 3) { // lane q writes component q
+        uint64_t f = q == 0 ? acc[0] : q == 1 ? acc[1] : acc[2];
+        for (int k = 0; k < 2; k++) {
+            const SortedForces &s = k == 0 ? s0 : s1;
+            const int slot = a < s.atoms ? s.slot_of[a] : -1;
+            if (slot >= 0) {
+                uint64_t *p = s.sorted + q * s.slots + slot;
+                f += *p;
+                *p = 0;
+            }
+        }
+        du_dx[a * 3 + q] = f;
     }
 }
 
@@ -229,38 +298,41 @@ void build_bonded_incidence(int A, const std::vector<const std::vector<int> *> &
     }
 }
 
-void launch_bonded_gather(const BondedIncidence &inc, const uint64_t *slots, uint64_t *du_dx, hipStream_t stream) {
+void launch_atom_forces(const BondedIncidence &inc, const uint64_t *slots, const SortedForces &s0,
+                        const SortedForces &s1, uint64_t *du_dx, hipStream_t stream) {
     if (inc.A == 0) {
         return;
     }
-    k_bonded_gather<<<ceil_div(inc.A, 256), 256, 0, stream>>>(inc, slots, du_dx);
+    k_atom_forces<<<ceil_div(inc.A, 256 / GATHER_LANES), 256, 0, stream>>>(inc, slots, s0, s1, du_dx);
+    TM_LAUNCH_CHECK();
+}
+
+void launch_bonded_all(const BondedSet &b, const double *x, const double *lambdas, const int *red_idx, uint64_t *du_dx,
+                       uint64_t *du_dl, uint64_t *u, hipStream_t stream) {
+    const int g1 = ceil_div(b.t[0].n, TERM_BLOCK);
+    const int g2 = g1 + ceil_div(b.t[1].n, TERM_BLOCK);
+    const int grid = g2 + ceil_div(b.t[2].n, TERM_BLOCK);
+    if (grid == 0) {
+        return;
+    }
+    k_bonded_all<<<grid, TERM_BLOCK, 0, stream>>>(b, g1, g2, x, lambdas, red_idx, du_dx, du_dl, u);
     TM_LAUNCH_CHECK();
 }
 
 void launch_bonded(BondedKind kind, const BondedTerms &t, const double *x, const double *lambdas, double lambda0,
                    const int *red_idx, uint64_t *du_dx, uint64_t *du_dp, uint64_t *du_dl, uint64_t *u,
-                   hipStream_t stream, bool dl_dp, uint64_t *slots) {
-    if (t.n == 0 || (!du_dx && !du_dp && !du_dl && !u && !slots)) {
+                   hipStream_t stream, bool dl_dp) {
+    if (t.n == 0 || (!du_dx && !du_dp && !du_dl && !u)) {
         return;
     }
     if (dl_dp && (du_dx || du_dl || u || !du_dp)) {
         throw Error("launch_bonded: the dl_dp mode writes du_dp only");
     }
-    const int grid = ceil_div(t.n, 128);
-    switch (kind) {
-    case BondedKind::Bond:
-        k_harmonic_bond<<<grid, 128, 0, stream>>>(t, x, lambdas, lambda0, red_idx, du_dx, du_dp, du_dl, u, dl_dp ? 1 : 0,
-                                                  slots);
-        break;
-    case BondedKind::Angle:
-        k_harmonic_angle<<<grid, 128, 0, stream>>>(t, x, lambdas, lambda0, red_idx, du_dx, du_dp, du_dl, u, dl_dp ? 1 : 0,
-                                                   slots);
-        break;
-    case BondedKind::Torsion:
-        k_periodic_torsion<<<grid, 128, 0, stream>>>(t, x, lambdas, lambda0, red_idx, du_dx, du_dp, du_dl, u, dl_dp ? 1 : 0,
-                                                     slots);
-        break;
-    }
+    auto kern = kind == BondedKind::Bond    ? k_bonded<BondedKind::Bond>
+                : kind == BondedKind::Angle ? k_bonded<BondedKind::Angle>
+                                            : k_bonded<BondedKind::Torsion>;
+    kern<<<ceil_div(t.n, TERM_BLOCK), TERM_BLOCK, 0, stream>>>(t, x, lambdas, lambda0, red_idx, du_dx, du_dp, du_dl, u,
+                                                              dl_dp ? 1 : 0, nullptr);
     TM_LAUNCH_CHECK();
 }
 

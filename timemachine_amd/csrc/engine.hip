@@ -798,6 +798,8 @@ struct Engine::Impl {
                        b_dvol.ptr,     b_lscale.ptr,   b_r2.ptr,       b_u_before.ptr, b_u_after.ptr};
     }
 
+    // Energies and forces of every system: writes ddx (all of its 3 A words), adds
+    // to ddl and uu; each may be null.
     void eval(const double *xp, const double *boxp, uint64_t *ddx, uint64_t *ddl, uint64_t *uu, hipStream_t st,
               int tile_grid, const double *lamp = nullptr) {
         if (!lamp) {
@@ -806,35 +808,40 @@ struct Engine::Impl {
         if (has_nb) {
             nb.prepare(xp, nb_params.ptr, nb_params1.n ? nb_params1.ptr : nullptr, boxp, nb_plane.ptr, nb_offset.ptr,
                        lamp, 0.0, st);
-            nb.compute(boxp, ddx, nullptr, ddl, uu, st, tile_grid);
+            nb.compute(boxp, ddx, nullptr, ddl, uu, st, tile_grid, true);
         }
         if (has_ig) {
             ig.prepare(xp, ig_params.ptr, ig_params1.n ? ig_params1.ptr : nullptr, boxp, ig_plane.ptr, ig_offset.ptr,
                        lamp, 0.0, st);
-            ig.compute(boxp, ddx, nullptr, ddl, uu, st, tile_grid);
+            ig.compute(boxp, ddx, nullptr, ddl, uu, st, tile_grid, true);
         }
-        const bool gather = bt_gather && ddx;
         for (int neg = 0; neg < 2; neg++) {
             if (pl_n[neg] == 0) {
                 continue;
             }
             PairListArgs a = pl_args(neg, xp, boxp);
             a.lambdas = lamp;
-            if (gather) {
+            if (ddx) {
                 a.slots = bt_slots.ptr + static_cast<size_t>(bt_slot0[3 + neg]) * 3;
             }
             launch_pair_list(a, ddx, nullptr, ddl, uu, st);
         }
-        for (int k = 0; k < 3; k++) {
-            if (bt_n[k] == 0) {
-                continue;
+        if ((ddx || ddl || uu) && bt_n[0] + bt_n[1] + bt_n[2] > 0) {
+            BondedSet b;
+            for (int k = 0; k < 3; k++) {
+                b.t[k] = {bt_n[k], bt_idx[k].ptr, bt_params[k].ptr, bt_mult[k].ptr, bt_offset[k].ptr, bt_sys[k].ptr};
+                b.slots[k] = ddx ? bt_slots.ptr + static_cast<size_t>(bt_slot0[k]) * 3 : nullptr;
             }
-            BondedTerms t{bt_n[k], bt_idx[k].ptr, bt_params[k].ptr, bt_mult[k].ptr, bt_offset[k].ptr, bt_sys[k].ptr};
-            launch_bonded(static_cast<BondedKind>(k), t, xp, lamp, 0.0, red_idx.ptr, gather ? nullptr : ddx, nullptr,
-                          ddl, uu, st, false, gather ? bt_slots.ptr + static_cast<size_t>(bt_slot0[k]) * 3 : nullptr);
+            launch_bonded_all(b, xp, lamp, red_idx.ptr, nullptr, ddl, uu, st);
         }
-        if (gather) {
-            launch_bonded_gather(BondedIncidence{A, bt_inc_off.ptr, bt_inc_items.ptr}, bt_slots.ptr, ddx, st);
+        if (ddx) {
+            auto sums = [](bool has, const NbState &n) {
+                return has ? SortedForces{n.sorted_acc.ptr, static_cast<size_t>(n.total_slots), n.slot_of.ptr,
+                                          static_cast<int>(n.slot_of.n)}
+                           : SortedForces{nullptr, 0, nullptr, 0};
+            };
+            launch_atom_forces(BondedIncidence{A, bt_gather ? bt_inc_off.ptr : nullptr, bt_inc_items.ptr},
+                               bt_slots.ptr, sums(has_nb, nb), sums(has_ig, ig), ddx, st);
         }
     }
 
@@ -1405,11 +1412,9 @@ void Engine::run(int n_steps, const double *lambda_sched, int du_dl_interval, in
             k_set_lambda<<<ceil_div(S_, 64), 64, 0, stream_>>>(S_, sched.ptr, n_steps, I.run_step.ptr, I.lam.ptr);
             TM_LAUNCH_CHECK();
         }
-        launch_fill_u64(I.du_dx.ptr, static_cast<size_t>(A_) * 3, 0, stream_);
         if (resolve_now) {
             // the move set up at the end of the previous step
             const BaroDev b = I.baro_dev();
-            launch_fill_u64(dx_trial.ptr, static_cast<size_t>(A_) * 3, 0, stream_);
             launch_fill_u64(dl_trial.ptr, S_, 0, stream_);
             I.eval(I.x.ptr, I.box.ptr, I.du_dx.ptr, dl_buf, I.b_u_before.ptr, stream_, tile_grid);
             if (I.nmol_total > 0) {
@@ -1900,7 +1905,6 @@ void Engine::adjoint_backward(const double *dl_bar, double *grad_out, double *x0
     };
     // one step of run() without barostat, frames or observer (the same launches)
     auto plain_step = [&]() {
-        launch_fill_u64(I.du_dx.ptr, n3, 0, stream_);
         I.eval(I.x.ptr, I.box.ptr, I.du_dx.ptr, I.du_dl_buf.ptr, nullptr, stream_, tile_grid);
         k_langevin<<<gA, TPB, 0, stream_>>>(A_, I.atom_sys.ptr, I.d_atom0.ptr, I.step.ptr, I.seed.ptr, I.ca.ptr,
                                             I.dt.ptr, I.cbs.ptr, I.ccs.ptr, I.du_dx.ptr, I.x.ptr, I.v.ptr,
@@ -2034,7 +2038,6 @@ void Engine::fire_minimize(int n_sched, const double *lambda_sched, const int *a
     const int gA = ceil_div(std::max(A3, 1), TPB);
     k_fire_state_init<<<ceil_div(S_, 64), 64, 0, stream_>>>(S_, dt.ptr, alpha.ptr, npos.ptr);
     TM_LAUNCH_CHECK();
-    launch_fill_u64(I.du_dx.ptr, A3, 0, stream_);
     I.eval(I.x.ptr, I.box.ptr, I.du_dx.ptr, nullptr, nullptr, stream_, tile_grid, d_sched.ptr);
     k_fire_init<<<gA, TPB, 0, stream_>>>(A3, I.atom_sys.ptr, d_act.ptr, I.du_dx.ptr, fv.ptr, ff.ptr);
     TM_LAUNCH_CHECK();
@@ -2051,7 +2054,6 @@ void Engine::fire_minimize(int n_sched, const double *lambda_sched, const int *a
             TM_HIP_CHECK(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
             k_fire_move<<<gA, TPB, 0, stream_>>>(A3, I.atom_sys.ptr, d_act.ptr, dt.ptr, fv.ptr, ff.ptr, I.x.ptr);
             TM_LAUNCH_CHECK();
-            launch_fill_u64(I.du_dx.ptr, A3, 0, stream_);
             k_fire_lambda<<<ceil_div(S_, 64), 64, 0, stream_>>>(S_, n_sched, d_sched.ptr, done.ptr, lam_cur.ptr);
             TM_LAUNCH_CHECK();
             I.eval(I.x.ptr, I.box.ptr, I.du_dx.ptr, nullptr, nullptr, stream_, tile_grid, lam_cur.ptr);
@@ -2079,7 +2081,6 @@ void Engine::fire_minimize(int n_sched, const double *lambda_sched, const int *a
 
 void Engine::max_force(double *out, bool raise) {
     Impl &I = *impl_;
-    launch_fill_u64(I.du_dx.ptr, A_ * 3, 0, stream_);
     I.eval(I.x.ptr, I.box.ptr, I.du_dx.ptr, nullptr, nullptr, stream_, tile_grid);
     DeviceArray<double> d(S_);
     k_max_force<<<S_, 256, 0, stream_>>>(I.d_atom0.ptr, I.d_natoms.ptr, I.du_dx.ptr, d.ptr);

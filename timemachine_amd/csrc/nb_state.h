@@ -150,6 +150,7 @@ struct NbState {
     // [total_blocks * NB_MAX_PIECES] (empty for views: one piece)
     DeviceArray<uint32_t> piece_buf;
     DeviceArray<int> piece_cnt;
+    DeviceArray<int> slot_of; // [sum n_atoms] sorted slot of each global atom, -1: none (empty for views)
     // [6 * total_slots] the tiles' sums of force and parameter derivatives by slot,
     // zero between launches (empty for views: tiles add to the atoms)
     DeviceArray<uint64_t> sorted_acc;
@@ -205,6 +206,8 @@ struct NbState {
 
     // Pair kernel over all tiles of all systems. Outputs are accumulated:
     //   du_dx [*, 3], du_dp [*, 3] (rows atom0 + i), du_dl / u [red_idx].
+    // keep_sorted: the force sums stay in sorted_acc (non-null du_dx only says
+    // that forces are wanted) and the caller takes and clears them.
     void compute(
         const double *boxes,
         uint64_t *du_dx,
@@ -212,7 +215,8 @@ struct NbState {
         uint64_t *du_dl,
         uint64_t *u,
         hipStream_t stream,
-        int grid_override = 0) const;
+        int grid_override = 0,
+        bool keep_sorted = false) const;
 
     void add_sorted(uint64_t *du_dx, uint64_t *du_dp, hipStream_t stream) const; // sorted_acc to the outputs
 

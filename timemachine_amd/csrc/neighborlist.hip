@@ -351,6 +351,8 @@ __global__ void k_gather(
     const double *__restrict__ lambdas,
     const double lambda0,
     const uint32_t *__restrict__ perm,
+    const int *__restrict__ rebuild,
+    int *__restrict__ slot_of,
     double4 *__restrict__ pos,
     float4 *__restrict__ par,
     float4 *__restrict__ dpar) {
@@ -370,6 +372,9 @@ __global__ void k_gather(
         return;
     }
     const int g = S.atom0 + static_cast<int>(atom);
+    if (slot_of && rebuild[s]) {
+        slot_of[g] = S.slot0 + slot;
+    }
     const double lam = lambdas ? lambdas[s] : lambda0;
     const int pl = plane ? plane[g] : 0;
     const int of = offset ? offset[g] : 0;
@@ -1113,6 +1118,8 @@ void NbState::init(const std::vector<NbSys> &sys_in, const std::vector<int> &sub
     bb_ext.alloc(total_blocks);
     piece_buf.alloc(static_cast<size_t>(total_blocks) * NB_MAX_PIECES * TILE);
     piece_cnt.alloc(static_cast<size_t>(total_blocks) * NB_MAX_PIECES);
+    slot_of.alloc(std::max(total_atoms_end, 1));
+    launch_fill_i32(slot_of.ptr, slot_of.n, -1, 0);
     sorted_acc.alloc(static_cast<size_t>(total_slots) * 6);
     red_slots.alloc(static_cast<size_t>(S) * NB_RED_SLOTS);
     nblist_x.alloc(static_cast<size_t>(total_atoms_end) * 3);
@@ -1190,7 +1197,8 @@ void NbState::build_only(const double *x, const double *boxes, hipStream_t strea
                                           nblist_box.ptr, tile_count.ptr);
     TM_LAUNCH_CHECK();
     k_gather<<<dim3(ceil_div(max_slots, 256), S), 256, 0, stream>>>(sys.ptr, x, nullptr, nullptr, nullptr, nullptr,
-                                                                    nullptr, nullptr, 0.0, perm.ptr, pos.ptr, par.ptr, nullptr);
+                                                                    nullptr, nullptr, 0.0, perm.ptr, rebuild.ptr, nullptr, pos.ptr, par.ptr,
+                                                                    nullptr);
     TM_LAUNCH_CHECK();
     k_block_bounds<<<dim3(ceil_div(max_blocks, 4), S), 256, 0, stream>>>(sys.ptr, boxes, rebuild.ptr, pos.ptr,
                                                                          bb_ctr.ptr, bb_ext.ptr);
@@ -1228,8 +1236,8 @@ void NbState::prepare(
                                           nblist_box.ptr, tile_count.ptr);
     TM_LAUNCH_CHECK();
     k_gather<<<dim3(ceil_div(max_slots, 256), S), 256, 0, stream>>>(
-        sys.ptr, x, boxes, params, params1, plane, offset, lambdas, lambda0, perm.ptr, pos.ptr, par.ptr,
-        any_interp ? dpar.ptr : nullptr);
+        sys.ptr, x, boxes, params, params1, plane, offset, lambdas, lambda0, perm.ptr, rebuild.ptr, slot_of.ptr, pos.ptr,
+        par.ptr, any_interp ? dpar.ptr : nullptr);
     TM_LAUNCH_CHECK();
     k_block_bounds<<<dim3(ceil_div(max_blocks, 4), S), 256, 0, stream>>>(sys.ptr, boxes, rebuild.ptr, pos.ptr,
                                                                          bb_ctr.ptr, bb_ext.ptr);

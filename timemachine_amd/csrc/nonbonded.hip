@@ -1094,7 +1094,8 @@ void NbState::compute(
     uint64_t *du_dl,
     uint64_t *u,
     hipStream_t stream,
-    int grid_override) const {
+    int grid_override,
+    bool keep_sorted) const {
     const int idx = kernel_index(du_dx, du_dp, du_dl, u);
     if (idx == 0) {
         return;
@@ -1105,7 +1106,7 @@ void NbState::compute(
                                         par.ptr, any_interp ? dpar.ptr : nullptr, boxes, bb_ctr.ptr, bb_ext.ptr,
                                         status.ptr, sorted_acc.ptr, total_slots, red_slots.ptr, du_dx, du_dp, du_dl, u);
     TM_LAUNCH_CHECK();
-    add_sorted(du_dx, du_dp, stream);
+    add_sorted(keep_sorted ? nullptr : du_dx, du_dp, stream);
 }
 
 void launch_pair_list(
