@@ -19,14 +19,41 @@ namespace {
 constexpr double BARO_AVOGADRO = 6.0221367e23;
 constexpr double BARO_BOLTZ = 0.008314462618;
 
+// lambda of run step r (past the end: the last step's)
+__device__ __forceinline__ double sched_lambda(const double *sched, int s, int n_steps, int r) {
+    return sched[static_cast<size_t>(s) * n_steps + (r < n_steps ? r : n_steps - 1)];
+}
+
 __global__ void k_set_lambda(int S, const double *__restrict__ sched, int n_steps, const int *__restrict__ run_step,
                              double *__restrict__ lam) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= S) {
         return;
     }
-    const int r = run_step[s];
-    lam[s] = sched[static_cast<size_t>(s) * n_steps + (r < n_steps ? r : n_steps - 1)];
+    lam[s] = sched_lambda(sched, s, n_steps, run_step[s]);
+}
+
+// Where the frames of a run go (frames null: none from this launch).
+struct FrameStore {
+    double *frames;
+    const int *natoms, *run_step;
+    int interval, F;
+};
+
+// Atom a's coordinates into the frame of the step that is being taken, if due.
+__device__ __forceinline__ void store_frame(const FrameStore &o, int a, int s, int a0, const double *x) {
+    const int r = o.run_step[s] + 1;
+    if (r % o.interval != 0) {
+        return;
+    }
+    const int f = r / o.interval - 1;
+    if (f >= o.F) {
+        return;
+    }
+    const size_t dst = static_cast<size_t>(o.F) * a0 * 3 + (static_cast<size_t>(f) * o.natoms[s] + (a - a0)) * 3;
+    o.frames[dst + 0] = x[0];
+    o.frames[dst + 1] = x[1];
+    o.frames[dst + 2] = x[2];
 }
 
 // BAOAB rotated by half a step (integrator.cu:37-69, integrator.py:81-88):
@@ -41,7 +68,7 @@ __global__ void k_langevin(int A, const int *__restrict__ atom_sys, const int *_
                            const double *__restrict__ ca, const double *__restrict__ dt,
                            const double *__restrict__ cbs, const double *__restrict__ ccs,
                            const uint64_t *__restrict__ du_dx, double *__restrict__ x, double *__restrict__ v,
-                           int *__restrict__ sys_status) {
+                           int *__restrict__ sys_status, const FrameStore out) {
     const int a = blockIdx.x * blockDim.x + threadIdx.x;
     if (a >= A) {
         return;
@@ -58,6 +85,7 @@ __global__ void k_langevin(int A, const int *__restrict__ atom_sys, const int *_
     normal2(philox4x32_10(c1, k0, k1), z[2], z[3]);
     const double cb = cbs[a], cc = ccs[a], cas = ca[s], h = 0.5 * dt[s];
     int bad = 0;
+    double xs[3];
     for (int d = 0; d < 3; d++) {
         const uint64_t fx = du_dx[a * 3 + d];
         const int64_t fi = static_cast<int64_t>(fx);
@@ -69,7 +97,7 @@ __global__ void k_langevin(int A, const int *__restrict__ atom_sys, const int *_
         const double v_new = cas * v_mid + cc * z[d];
         v[a * 3 + d] = v_new;
         const double x_new = x[a * 3 + d] + h * (v_mid + v_new);
-        x[a * 3 + d] = x_new;
+        x[a * 3 + d] = xs[d] = x_new;
         if (!isfinite(x_new) || !isfinite(v_new)) {
             bad |= ENGINE_STATUS_NONFINITE;
         }
@@ -77,61 +105,19 @@ __global__ void k_langevin(int A, const int *__restrict__ atom_sys, const int *_
     if (bad) {
         atomicOr(sys_status + s, bad);
     }
+    if (out.frames) {
+        store_frame(out, a, s, atom0[s], xs);
+    }
 }
 
-// du_dl store, box frame store, per-system step counters.
-__global__ void k_step_end(int S, int64_t *__restrict__ step, int *__restrict__ run_step,
-                           uint64_t *__restrict__ du_dl_buf, int dl_interval, int K, uint64_t *__restrict__ du_dl_traj,
-                           int x_interval, int F, const double *__restrict__ box, double *__restrict__ box_frames) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= S) {
-        return;
-    }
-    const int r = run_step[s] + 1;
-    if (dl_interval > 0) {
-        if (r % dl_interval == 0) {
-            const int k = r / dl_interval - 1;
-            if (k < K) {
-                du_dl_traj[static_cast<size_t>(s) * K + k] = du_dl_buf[s];
-            }
-        }
-        du_dl_buf[s] = 0;
-    }
-    if (x_interval > 0 && r % x_interval == 0) {
-        const int f = r / x_interval - 1;
-        if (f < F) {
-            for (int d = 0; d < 9; d++) {
-                box_frames[(static_cast<size_t>(s) * F + f) * 9 + d] = box[s * 9 + d];
-            }
-        }
-    }
-    run_step[s] = r;
-    step[s] += 1;
-}
-
-// Frame store with an explicit per-system atom count table.
-__global__ void k_store_frames2(int A, const int *__restrict__ atom_sys, const int *__restrict__ atom0,
-                                const int *__restrict__ natoms, const int *__restrict__ run_step, int x_interval,
-                                int F, const double *__restrict__ x, double *__restrict__ frames) {
+// Frame store on its own, for steps whose coordinates change after the update.
+__global__ void k_store_frames(int A, const int *__restrict__ atom_sys, const int *__restrict__ atom0,
+                               const double *__restrict__ x, const FrameStore out) {
     const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= A) {
-        return;
+    if (a < A) {
+        const int s = atom_sys[a];
+        store_frame(out, a, s, atom0[s], x + a * 3);
     }
-    const int s = atom_sys[a];
-    const int r = run_step[s] + 1;
-    if (r % x_interval != 0) {
-        return;
-    }
-    const int f = r / x_interval - 1;
-    if (f >= F) {
-        return;
-    }
-    const int a0 = atom0[s];
-    const int ns = natoms[s];
-    const size_t dst = static_cast<size_t>(F) * a0 * 3 + (static_cast<size_t>(f) * ns + (a - a0)) * 3;
-    frames[dst + 0] = x[a * 3 + 0];
-    frames[dst + 1] = x[a * 3 + 1];
-    frames[dst + 2] = x[a * 3 + 2];
 }
 
 // Energies at other lambda windows: every system evaluates window w.
@@ -474,12 +460,8 @@ struct BaroDev {
 // not on the call counter, which only holds the phase within the interval: a
 // rebuilt engine (batch hand-over, set_pressure, set_interval) continues the
 // stream instead of repeating its first draws.
-__global__ void k_baro_setup(int S, BaroDev b, const int64_t *__restrict__ step, const double *__restrict__ box,
-                             double *__restrict__ box_after) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= S) {
-        return;
-    }
+__device__ __forceinline__ void baro_setup(int s, const BaroDev &b, const int64_t *__restrict__ step,
+                                           const double *__restrict__ box, double *__restrict__ box_after) {
     b.trig[s] = 0;
     b.accept[s] = 0;
     b.u_before[s] = 0;
@@ -514,6 +496,62 @@ __global__ void k_baro_setup(int S, BaroDev b, const int64_t *__restrict__ step,
     box_after[s * 9 + 0] = box[s * 9 + 0] * ls;
     box_after[s * 9 + 4] = box[s * 9 + 4] * ls;
     box_after[s * 9 + 8] = box[s * 9 + 8] * ls;
+}
+
+__global__ void k_baro_setup(int S, BaroDev b, const int64_t *__restrict__ step, const double *__restrict__ box,
+                             double *__restrict__ box_after) {
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s < S) {
+        baro_setup(s, b, step, box, box_after);
+    }
+}
+
+// What a step's last launch does besides its counters: the next barostat move's
+// draws (box_after non-null) and the next step's lambda (sched non-null). Each
+// was a launch of its own before, 4.4 us in a graph for a few words of work.
+struct StepTail {
+    BaroDev baro;
+    double *box_after;
+    const double *sched;
+    int n_steps;
+    double *lam;
+};
+
+// du_dl store, box frame store, per-system step counters.
+__global__ void k_step_end(int S, int64_t *__restrict__ step, int *__restrict__ run_step,
+                           uint64_t *__restrict__ du_dl_buf, int dl_interval, int K, uint64_t *__restrict__ du_dl_traj,
+                           int x_interval, int F, const double *__restrict__ box, double *__restrict__ box_frames,
+                           const StepTail tail) {
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= S) {
+        return;
+    }
+    if (tail.box_after) {
+        baro_setup(s, tail.baro, step, box, tail.box_after);
+    }
+    const int r = run_step[s] + 1;
+    if (dl_interval > 0) {
+        if (r % dl_interval == 0) {
+            const int k = r / dl_interval - 1;
+            if (k < K) {
+                du_dl_traj[static_cast<size_t>(s) * K + k] = du_dl_buf[s];
+            }
+        }
+        du_dl_buf[s] = 0;
+    }
+    if (x_interval > 0 && r % x_interval == 0) {
+        const int f = r / x_interval - 1;
+        if (f < F) {
+            for (int d = 0; d < 9; d++) {
+                box_frames[(static_cast<size_t>(s) * F + f) * 9 + d] = box[s * 9 + d];
+            }
+        }
+    }
+    run_step[s] = r;
+    step[s] += 1;
+    if (tail.sched) {
+        tail.lam[s] = sched_lambda(tail.sched, s, tail.n_steps, r);
+    }
 }
 
 __global__ void k_baro_zero_centroids(int nmol_total, const int *__restrict__ mol_sys, const int *__restrict__ trig,
@@ -1407,11 +1445,14 @@ void Engine::run(int n_steps, const double *lambda_sched, int du_dl_interval, in
 
     const int TPB = 256;
     const int obs_k = I.obs_interval;
+    if (lambda_sched && n_steps > 0) { // the first step's; each step's last launch sets the next one's
+        k_set_lambda<<<ceil_div(S_, 64), 64, 0, stream_>>>(S_, sched.ptr, n_steps, I.run_step.ptr, I.lam.ptr);
+        TM_LAUNCH_CHECK();
+    }
     auto one_step = [&](bool baro_now, bool obs_now, bool u_now, bool defer_now, bool resolve_now) {
-        if (lambda_sched) {
-            k_set_lambda<<<ceil_div(S_, 64), 64, 0, stream_>>>(S_, sched.ptr, n_steps, I.run_step.ptr, I.lam.ptr);
-            TM_LAUNCH_CHECK();
-        }
+        // the move of this step is evaluated within it, after the update
+        const bool move_now = I.has_baro && baro_now && !defer_now;
+        const FrameStore frame_store{frames.ptr, I.d_natoms.ptr, I.run_step.ptr, x_interval, F};
         if (resolve_now) {
             // the move set up at the end of the previous step
             const BaroDev b = I.baro_dev();
@@ -1448,34 +1489,33 @@ void Engine::run(int n_steps, const double *lambda_sched, int du_dl_interval, in
         }
         k_langevin<<<ceil_div(A_, TPB), TPB, 0, stream_>>>(A_, I.atom_sys.ptr, I.d_atom0.ptr, I.step.ptr, I.seed.ptr,
                                                          I.ca.ptr, I.dt.ptr, I.cbs.ptr, I.ccs.ptr, I.du_dx.ptr,
-                                                         I.x.ptr, I.v.ptr, I.sys_status.ptr);
+                                                         I.x.ptr, I.v.ptr, I.sys_status.ptr,
+                                                         x_interval > 0 && !move_now ? frame_store : FrameStore{});
         TM_LAUNCH_CHECK();
-        if (I.has_baro) {
+        if (move_now) {
             const BaroDev b = I.baro_dev();
             k_baro_setup<<<ceil_div(S_, 64), 64, 0, stream_>>>(S_, b, I.step.ptr, I.box.ptr, I.box_after.ptr);
             TM_LAUNCH_CHECK();
-            if (baro_now && !defer_now) {
-                I.eval(I.x.ptr, I.box.ptr, nullptr, nullptr, I.b_u_before.ptr, stream_, tile_grid);
-                if (I.nmol_total > 0) {
-                    k_baro_zero_centroids<<<ceil_div(I.nmol_total, TPB), TPB, 0, stream_>>>(
-                        I.nmol_total, I.mol_sys.ptr, I.b_trig.ptr, I.centroids.ptr);
-                    TM_LAUNCH_CHECK();
-                    k_baro_centroids<<<ceil_div(I.G, TPB), TPB, 0, stream_>>>(I.G, I.g_atom.ptr, I.g_mol.ptr,
-                                                                           I.mol_sys.ptr, I.b_trig.ptr, I.x.ptr,
-                                                                           I.centroids.ptr);
-                    TM_LAUNCH_CHECK();
-                }
-                k_baro_rescale<<<ceil_div(A_, TPB), TPB, 0, stream_>>>(
-                    A_, I.atom_sys.ptr, I.atom_mol.ptr, I.mol_count.ptr, I.b_trig.ptr, I.b_lscale.ptr, I.box.ptr,
-                    I.centroids.ptr, I.x.ptr, I.x_after.ptr);
+            I.eval(I.x.ptr, I.box.ptr, nullptr, nullptr, I.b_u_before.ptr, stream_, tile_grid);
+            if (I.nmol_total > 0) {
+                k_baro_zero_centroids<<<ceil_div(I.nmol_total, TPB), TPB, 0, stream_>>>(
+                    I.nmol_total, I.mol_sys.ptr, I.b_trig.ptr, I.centroids.ptr);
                 TM_LAUNCH_CHECK();
-                I.eval(I.x_after.ptr, I.box_after.ptr, nullptr, nullptr, I.b_u_after.ptr, stream_, tile_grid);
-                k_baro_decide<<<ceil_div(S_, 64), 64, 0, stream_>>>(S_, b, I.box.ptr, I.box_after.ptr);
-                TM_LAUNCH_CHECK();
-                k_baro_apply<<<ceil_div(A_, TPB), TPB, 0, stream_>>>(A_, I.atom_sys.ptr, I.b_accept.ptr,
-                                                                   I.x_after.ptr, I.x.ptr);
+                k_baro_centroids<<<ceil_div(I.G, TPB), TPB, 0, stream_>>>(I.G, I.g_atom.ptr, I.g_mol.ptr,
+                                                                       I.mol_sys.ptr, I.b_trig.ptr, I.x.ptr,
+                                                                       I.centroids.ptr);
                 TM_LAUNCH_CHECK();
             }
+            k_baro_rescale<<<ceil_div(A_, TPB), TPB, 0, stream_>>>(
+                A_, I.atom_sys.ptr, I.atom_mol.ptr, I.mol_count.ptr, I.b_trig.ptr, I.b_lscale.ptr, I.box.ptr,
+                I.centroids.ptr, I.x.ptr, I.x_after.ptr);
+            TM_LAUNCH_CHECK();
+            I.eval(I.x_after.ptr, I.box_after.ptr, nullptr, nullptr, I.b_u_after.ptr, stream_, tile_grid);
+            k_baro_decide<<<ceil_div(S_, 64), 64, 0, stream_>>>(S_, b, I.box.ptr, I.box_after.ptr);
+            TM_LAUNCH_CHECK();
+            k_baro_apply<<<ceil_div(A_, TPB), TPB, 0, stream_>>>(A_, I.atom_sys.ptr, I.b_accept.ptr,
+                                                               I.x_after.ptr, I.x.ptr);
+            TM_LAUNCH_CHECK();
         }
         if (u_now) {
             // energies of the state after this step at every window (context.cu:139-233)
@@ -1488,15 +1528,24 @@ void Engine::run(int n_steps, const double *lambda_sched, int du_dl_interval, in
                 TM_LAUNCH_CHECK();
             }
         }
-        if (x_interval > 0) {
-            k_store_frames2<<<ceil_div(A_, TPB), TPB, 0, stream_>>>(A_, I.atom_sys.ptr, I.d_atom0.ptr,
-                                                                  I.d_natoms.ptr, I.run_step.ptr, x_interval, F,
-                                                                  I.x.ptr, frames.ptr);
+        if (x_interval > 0 && move_now) {
+            k_store_frames<<<ceil_div(A_, TPB), TPB, 0, stream_>>>(A_, I.atom_sys.ptr, I.d_atom0.ptr, I.x.ptr,
+                                                                 frame_store);
             TM_LAUNCH_CHECK();
+        }
+        StepTail tail{};
+        if (I.has_baro && !move_now) {
+            tail.baro = I.baro_dev();
+            tail.box_after = I.box_after.ptr;
+        }
+        if (lambda_sched) {
+            tail.sched = sched.ptr;
+            tail.n_steps = n_steps;
+            tail.lam = I.lam.ptr;
         }
         k_step_end<<<ceil_div(S_, 64), 64, 0, stream_>>>(S_, I.step.ptr, I.run_step.ptr, I.du_dl_buf.ptr,
                                                         du_dl_interval, Kst, dl_ptr, x_interval, F, I.box.ptr,
-                                                        box_frames_ptr);
+                                                        box_frames_ptr, tail);
         TM_LAUNCH_CHECK();
     };
 
@@ -1908,10 +1957,10 @@ void Engine::adjoint_backward(const double *dl_bar, double *grad_out, double *x0
         I.eval(I.x.ptr, I.box.ptr, I.du_dx.ptr, I.du_dl_buf.ptr, nullptr, stream_, tile_grid);
         k_langevin<<<gA, TPB, 0, stream_>>>(A_, I.atom_sys.ptr, I.d_atom0.ptr, I.step.ptr, I.seed.ptr, I.ca.ptr,
                                             I.dt.ptr, I.cbs.ptr, I.ccs.ptr, I.du_dx.ptr, I.x.ptr, I.v.ptr,
-                                            I.sys_status.ptr);
+                                            I.sys_status.ptr, FrameStore{});
         TM_LAUNCH_CHECK();
         k_step_end<<<gS, 64, 0, stream_>>>(S_, I.step.ptr, I.run_step.ptr, I.du_dl_buf.ptr, 1, 0, nullptr, 0, 0,
-                                          I.box.ptr, nullptr);
+                                          I.box.ptr, nullptr, StepTail{});
         TM_LAUNCH_CHECK();
     };
     HvpTangent tan;
@@ -2274,7 +2323,7 @@ void Engine::profile(int reps, double *ms_out) {
     ms_out[3] = timed([&] {
         k_langevin<<<ceil_div(A_, 256), 256, 0, stream_>>>(A_, I.atom_sys.ptr, I.d_atom0.ptr, I.step.ptr, I.seed.ptr,
                                                          I.ca.ptr, I.dt.ptr, I.cbs.ptr, I.ccs.ptr, I.du_dx.ptr,
-                                                         xs.ptr, vs.ptr, scratch_status.ptr);
+                                                         xs.ptr, vs.ptr, scratch_status.ptr, FrameStore{});
     });
     TM_HIP_CHECK(hipStreamSynchronize(stream_));
     launch_fill_u64(I.du_dx.ptr, static_cast<size_t>(A_) * 3, 0, stream_);

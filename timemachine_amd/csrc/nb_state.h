@@ -134,6 +134,7 @@ struct NbState {
     DeviceArray<int> status;      // [S]
     DeviceArray<int> tile_count;  // [S * NB_TILE_LANES]
     DeviceArray<int> tile_prefix; // [S + 1]
+    DeviceArray<int> order_done;  // [1] workgroups of the tile order that are done, 0 between launches (empty for views)
     DeviceArray<int> tile_row;    // [total_tiles]
     DeviceArray<int> tile_order;  // [total_tiles] per system: local tile indices grouped by row block
     DeviceArray<uint32_t> tile_atoms; // [total_tiles * 64]

@@ -335,15 +335,46 @@ __global__ __launch_bounds__(SORT_THREADS) void k_sort(
     }
 }
 
+// Bounding box of block b, one wave: every atom imaged next to the block's first
+// atom (a valid periodic box for any block narrower than half the box).
+__device__ __forceinline__ void block_bounds(const NbSys &S, int b, float4 p, const double *box, float4 *bb_ctr,
+                                             float4 *bb_ext) {
+    const int lane = threadIdx.x & 63;
+    const float bx = static_cast<float>(box[0]);
+    const float by = static_cast<float>(box[4]);
+    const float bz = static_cast<float>(box[8]);
+    const float ibx = 1.0f / bx;
+    const float iby = 1.0f / by;
+    const float ibz = 1.0f / bz;
+    const float rx = __shfl(p.x, 0, 64), ry = __shfl(p.y, 0, 64), rz = __shfl(p.z, 0, 64);
+    float px = rx, py = ry, pz = rz;
+    if (b * TILE + lane < nb_block_end(S, b)) {
+        px = rx + min_image_f(p.x - rx, bx, ibx);
+        py = ry + min_image_f(p.y - ry, by, iby);
+        pz = rz + min_image_f(p.z - rz, bz, ibz);
+    }
+    const float lox = wave_min(px), hix = wave_max(px);
+    const float loy = wave_min(py), hiy = wave_max(py);
+    const float loz = wave_min(pz), hiz = wave_max(pz);
+    if (lane == 0) {
+        bb_ctr[S.block0 + b] = make_float4(0.5f * (lox + hix), 0.5f * (loy + hiy), 0.5f * (loz + hiz), 0.f);
+        bb_ext[S.block0 + b] = make_float4(0.5f * (hix - lox), 0.5f * (hiy - loy), 0.5f * (hiz - loz), 0.f);
+    }
+}
+
 // grid (ceil(max_slots / 256), S): sorted FP32 coordinates and parameters.
 // w = (plane + offset * lambda) * cutoff and dw/dlambda = offset * cutoff, in
 // f64 before rounding to FP32 (kernels/k_lambda_transformer_jit.cuh:25-55 with
-// the identity transform). With boxes the coordinates are wrapped onto the box's
-// grid (BoxAxis), as the pair kernels expect them; without, they are copied.
+// the identity transform). With wrap the coordinates are wrapped onto the box's
+// grid (BoxAxis), as the pair kernels expect them; without, they are copied. In
+// systems that rebuild, each wave also leaves its block's bounding box (as a
+// launch of its own that read the coordinates again, this took 4.4 us of every
+// graph replay, rebuild or not).
 __global__ void k_gather(
     const NbSys *__restrict__ sys,
     const double *__restrict__ x,
     const double *__restrict__ boxes,
+    const int wrap,
     const double *__restrict__ params,
     const double *__restrict__ params1,
     const int *__restrict__ plane,
@@ -355,7 +386,9 @@ __global__ void k_gather(
     int *__restrict__ slot_of,
     double4 *__restrict__ pos,
     float4 *__restrict__ par,
-    float4 *__restrict__ dpar) {
+    float4 *__restrict__ dpar,
+    float4 *__restrict__ bb_ctr,
+    float4 *__restrict__ bb_ext) {
     const int s = blockIdx.y;
     const NbSys S = sys[s];
     const int slot = blockIdx.x * blockDim.x + threadIdx.x;
@@ -363,30 +396,36 @@ __global__ void k_gather(
         return;
     }
     const uint32_t atom = perm[S.slot0 + slot];
-    if (atom == NB_INVALID) {
-        pos[S.slot0 + slot] = make_double4(0.0, 0.0, 0.0, 0.0);
+    const bool valid = atom != NB_INVALID;
+    const bool built = rebuild[s] != 0;
+    const int g = valid ? S.atom0 + static_cast<int>(atom) : 0;
+    const double lam = lambdas ? lambdas[s] : lambda0;
+    const int of = valid && offset ? offset[g] : 0;
+    const double dw_dl = of * S.cutoff_d;
+    double4 p4 = make_double4(0.0, 0.0, 0.0, 0.0);
+    if (valid) {
+        const int pl = plane ? plane[g] : 0;
+        p4 = make_double4(x[g * 3 + 0], x[g * 3 + 1], x[g * 3 + 2], (pl + of * lam) * S.cutoff_d);
+        if (wrap) {
+            p4.x = BoxAxis(boxes[s * 9 + 0]).wrap(p4.x);
+            p4.y = BoxAxis(boxes[s * 9 + 4]).wrap(p4.y);
+            p4.z = BoxAxis(boxes[s * 9 + 8]).wrap(p4.z);
+        }
+        if (slot_of && built) {
+            slot_of[g] = S.slot0 + slot;
+        }
+    }
+    pos[S.slot0 + slot] = p4;
+    if (built) { // the whole wave
+        block_bounds(S, slot / TILE, to_f32(p4), boxes + s * 9, bb_ctr, bb_ext);
+    }
+    if (!valid) {
         par[S.slot0 + slot] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (dpar) {
             dpar[S.slot0 + slot] = make_float4(0.f, 0.f, 0.f, 0.f);
         }
         return;
     }
-    const int g = S.atom0 + static_cast<int>(atom);
-    if (slot_of && rebuild[s]) {
-        slot_of[g] = S.slot0 + slot;
-    }
-    const double lam = lambdas ? lambdas[s] : lambda0;
-    const int pl = plane ? plane[g] : 0;
-    const int of = offset ? offset[g] : 0;
-    const double w = (pl + of * lam) * S.cutoff_d;
-    const double dw_dl = of * S.cutoff_d;
-    double4 p4 = make_double4(x[g * 3 + 0], x[g * 3 + 1], x[g * 3 + 2], w);
-    if (boxes) {
-        p4.x = BoxAxis(boxes[s * 9 + 0]).wrap(p4.x);
-        p4.y = BoxAxis(boxes[s * 9 + 4]).wrap(p4.y);
-        p4.z = BoxAxis(boxes[s * 9 + 8]).wrap(p4.z);
-    }
-    pos[S.slot0 + slot] = p4;
     if (params) {
         if (S.interp && params1) {
             // parameter interpolation with the identity transform
@@ -424,50 +463,6 @@ __global__ void k_split_interpolated_du_dp(int N, double lambda, const uint64_t 
     const double g = fixed_to_double(src[i * 3 + c], scale);
     dst[i * 3 + c] += f64_to_fixed((1.0 - lambda) * g, scale);
     dst[(N + i) * 3 + c] += f64_to_fixed(lambda * g, scale);
-}
-
-// grid (ceil(max_blocks / 4), S), 256 threads: one wave per 64-atom block.
-// Bounding box of the block with every atom imaged next to the block's first
-// atom (a valid periodic box for any block narrower than half the box).
-__global__ __launch_bounds__(256) void k_block_bounds(
-    const NbSys *__restrict__ sys,
-    const double *__restrict__ boxes,
-    const int *__restrict__ rebuild,
-    const double4 *__restrict__ pos,
-    float4 *__restrict__ bb_ctr,
-    float4 *__restrict__ bb_ext) {
-    const int s = blockIdx.y;
-    if (!rebuild[s]) {
-        return;
-    }
-    const NbSys S = sys[s];
-    const int b = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (b >= S.nblocks) {
-        return;
-    }
-    const int lane = threadIdx.x & 63;
-    const float bx = static_cast<float>(boxes[s * 9 + 0]);
-    const float by = static_cast<float>(boxes[s * 9 + 4]);
-    const float bz = static_cast<float>(boxes[s * 9 + 8]);
-    const float ibx = 1.0f / bx;
-    const float iby = 1.0f / by;
-    const float ibz = 1.0f / bz;
-    const float4 ref = to_f32(pos[S.slot0 + b * TILE]);
-    const int slot = b * TILE + lane;
-    float px = ref.x, py = ref.y, pz = ref.z;
-    if (slot < nb_block_end(S, b)) {
-        const float4 p = to_f32(pos[S.slot0 + slot]);
-        px = ref.x + min_image_f(p.x - ref.x, bx, ibx);
-        py = ref.y + min_image_f(p.y - ref.y, by, iby);
-        pz = ref.z + min_image_f(p.z - ref.z, bz, ibz);
-    }
-    const float lox = wave_min(px), hix = wave_max(px);
-    const float loy = wave_min(py), hiy = wave_max(py);
-    const float loz = wave_min(pz), hiz = wave_max(pz);
-    if (lane == 0) {
-        bb_ctr[S.block0 + b] = make_float4(0.5f * (lox + hix), 0.5f * (loy + hiy), 0.5f * (loz + hiz), 0.f);
-        bb_ext[S.block0 + b] = make_float4(0.5f * (hix - lox), 0.5f * (hiy - loy), 0.5f * (hiz - loz), 0.f);
-    }
 }
 
 __device__ __forceinline__ float box_gap(float d, float ext, float b, float ib) {
@@ -804,14 +799,8 @@ __global__ __launch_bounds__(256) void k_merge_pieces(
 // blocks than the LDS histogram holds list them counter by counter.
 constexpr int ORDER_ROWS = 4096;
 
-__global__ __launch_bounds__(256) void k_tile_order(
-    const NbSys *__restrict__ sys, const int *__restrict__ rebuild, const int *__restrict__ tile_count,
-    const int *__restrict__ tile_row, int *__restrict__ tile_order) {
-    const int s = blockIdx.x;
-    if (!rebuild[s]) {
-        return;
-    }
-    const NbSys S = sys[s];
+__device__ __forceinline__ void order_tiles(const NbSys &S, const int s, const int *__restrict__ tile_count,
+                                            const int *__restrict__ tile_row, int *__restrict__ tile_order) {
     const int rb = S.row_blocks;
     const int t = threadIdx.x;
     int *order = tile_order + S.tile0;
@@ -884,12 +873,10 @@ __global__ __launch_bounds__(256) void k_tile_order(
     }
 }
 
-// One workgroup: valid tiles of each system (counts limited to the capacity),
-// exclusive prefix over systems
-// (tile_prefix[S] = total), clear the rebuild flags.
-__global__ __launch_bounds__(256) void k_tile_prefix(
-    const NbSys *__restrict__ sys, int S, int *__restrict__ tile_count, int *__restrict__ tile_prefix,
-    int *__restrict__ rebuild) {
+// Valid tiles of each system (counts limited to the capacity), exclusive prefix
+// over systems (tile_prefix[S] = total), clear the rebuild flags; one workgroup.
+__device__ __forceinline__ void prefix_tiles(const NbSys *__restrict__ sys, int S, const int *__restrict__ tile_count,
+                                             int *__restrict__ tile_prefix, int *__restrict__ rebuild) {
     __shared__ int part[256];
     const int t = threadIdx.x;
     const int per = (S + 255) / 256;
@@ -929,6 +916,35 @@ __global__ __launch_bounds__(256) void k_tile_prefix(
             rebuild[s] = 0;
         }
     }
+}
+
+// One workgroup per system orders its tiles if they were rebuilt; the last one to
+// finish then does the prefix over all of them (done counts the workgroups and
+// returns to 0; one system needs no count). In a launch of its own the prefix
+// took 4.2 us of every graph replay.
+__global__ __launch_bounds__(256) void k_tile_order(const NbSys *__restrict__ sys, int S, int *__restrict__ rebuild,
+                                                    const int *__restrict__ tile_count,
+                                                    const int *__restrict__ tile_row, int *__restrict__ tile_order,
+                                                    int *__restrict__ tile_prefix, int *__restrict__ done) {
+    const int s = blockIdx.x;
+    if (rebuild[s]) {
+        order_tiles(sys[s], s, tile_count, tile_row, tile_order);
+    }
+    __syncthreads(); // every thread has read the flag
+    if (S > 1) {
+        __shared__ int last;
+        if (threadIdx.x == 0) {
+            last = atomicAdd(done, 1) == S - 1;
+        }
+        __syncthreads();
+        if (!last) {
+            return;
+        }
+        if (threadIdx.x == 0) {
+            *done = 0;
+        }
+    }
+    prefix_tiles(sys, S, tile_count, tile_prefix, rebuild);
 }
 
 } // namespace
@@ -1098,6 +1114,7 @@ void NbState::init(const std::vector<NbSys> &sys_in, const std::vector<int> &sub
     status.alloc(S);
     tile_count.alloc(static_cast<size_t>(S) * NB_TILE_LANES);
     tile_prefix.alloc(S + 1);
+    order_done.alloc(1);
     tile_row.alloc(total_tiles);
     tile_order.alloc(total_tiles);
     tile_atoms.alloc(static_cast<size_t>(total_tiles) * TILE);
@@ -1127,6 +1144,7 @@ void NbState::init(const std::vector<NbSys> &sys_in, const std::vector<int> &sub
     status.zero();
     tile_count.zero();
     tile_prefix.zero();
+    order_done.zero();
     sorted_acc.zero();
     red_slots.zero();
     nblist_x.zero();
@@ -1196,17 +1214,13 @@ void NbState::build_only(const double *x, const double *boxes, hipStream_t strea
     k_sort<<<S, SORT_THREADS, 0, stream>>>(sys.ptr, subset.ptr, x, boxes, rebuild.ptr, keys.ptr, perm.ptr, nblist_x.ptr,
                                           nblist_box.ptr, tile_count.ptr);
     TM_LAUNCH_CHECK();
-    k_gather<<<dim3(ceil_div(max_slots, 256), S), 256, 0, stream>>>(sys.ptr, x, nullptr, nullptr, nullptr, nullptr,
-                                                                    nullptr, nullptr, 0.0, perm.ptr, rebuild.ptr, nullptr, pos.ptr, par.ptr,
-                                                                    nullptr);
-    TM_LAUNCH_CHECK();
-    k_block_bounds<<<dim3(ceil_div(max_blocks, 4), S), 256, 0, stream>>>(sys.ptr, boxes, rebuild.ptr, pos.ptr,
-                                                                         bb_ctr.ptr, bb_ext.ptr);
+    k_gather<<<dim3(ceil_div(max_slots, 256), S), 256, 0, stream>>>(
+        sys.ptr, x, boxes, 0, nullptr, nullptr, nullptr, nullptr, nullptr, 0.0, perm.ptr, rebuild.ptr, nullptr, pos.ptr,
+        par.ptr, nullptr, bb_ctr.ptr, bb_ext.ptr);
     TM_LAUNCH_CHECK();
     find_tiles(boxes, stream);
-    k_tile_order<<<S, 256, 0, stream>>>(sys.ptr, rebuild.ptr, tile_count.ptr, tile_row.ptr, tile_order.ptr);
-    TM_LAUNCH_CHECK();
-    k_tile_prefix<<<1, 256, 0, stream>>>(sys.ptr, S, tile_count.ptr, tile_prefix.ptr, rebuild.ptr);
+    k_tile_order<<<S, 256, 0, stream>>>(sys.ptr, S, rebuild.ptr, tile_count.ptr, tile_row.ptr, tile_order.ptr,
+                                        tile_prefix.ptr, order_done.ptr);
     TM_LAUNCH_CHECK();
 }
 
@@ -1236,16 +1250,12 @@ void NbState::prepare(
                                           nblist_box.ptr, tile_count.ptr);
     TM_LAUNCH_CHECK();
     k_gather<<<dim3(ceil_div(max_slots, 256), S), 256, 0, stream>>>(
-        sys.ptr, x, boxes, params, params1, plane, offset, lambdas, lambda0, perm.ptr, rebuild.ptr, slot_of.ptr, pos.ptr,
-        par.ptr, any_interp ? dpar.ptr : nullptr);
-    TM_LAUNCH_CHECK();
-    k_block_bounds<<<dim3(ceil_div(max_blocks, 4), S), 256, 0, stream>>>(sys.ptr, boxes, rebuild.ptr, pos.ptr,
-                                                                         bb_ctr.ptr, bb_ext.ptr);
+        sys.ptr, x, boxes, 1, params, params1, plane, offset, lambdas, lambda0, perm.ptr, rebuild.ptr, slot_of.ptr,
+        pos.ptr, par.ptr, any_interp ? dpar.ptr : nullptr, bb_ctr.ptr, bb_ext.ptr);
     TM_LAUNCH_CHECK();
     find_tiles(boxes, stream);
-    k_tile_order<<<S, 256, 0, stream>>>(sys.ptr, rebuild.ptr, tile_count.ptr, tile_row.ptr, tile_order.ptr);
-    TM_LAUNCH_CHECK();
-    k_tile_prefix<<<1, 256, 0, stream>>>(sys.ptr, S, tile_count.ptr, tile_prefix.ptr, rebuild.ptr);
+    k_tile_order<<<S, 256, 0, stream>>>(sys.ptr, S, rebuild.ptr, tile_count.ptr, tile_row.ptr, tile_order.ptr,
+                                        tile_prefix.ptr, order_done.ptr);
     TM_LAUNCH_CHECK();
 }
 

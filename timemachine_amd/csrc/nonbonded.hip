@@ -371,7 +371,7 @@ __device__ __forceinline__ uint64_t item_mask(uint64_t m0, uint64_t m1) {
 // image differs by a multiple of L, so |a_j - a_i| >= L - cutoff > L / 2 + e,
 // which a_j - a_i cannot reach; pass 2 then needs no image (9 of ~75
 // instructions a pair). c and e come from the block's bounding box of the last
-// neighborlist build (k_block_bounds, FP32): since then the box is unchanged
+// neighborlist build (block_bounds, FP32): since then the box is unchanged
 // and no atom has moved more than padding / 2, so every row atom is within the
 // box's half-extent + padding / 2 of its centre, plus 1e-4 nm for the FP32
 // rounding of the build. Otherwise ("image", boxes under ~3.4 nm) the screen
