@@ -8,6 +8,7 @@
 #pragma once
 
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -27,6 +28,20 @@ enum class PotKind {
     PeriodicTorsion,
     Summed,
     Fanout
+};
+
+// Device workspace and pinned staging of a potential's host calls, kept between
+// calls and freed with the potential. As large as its largest call.
+struct HostBuffer {
+    std::mutex m;
+    uint64_t *dev = nullptr, *pin = nullptr;
+    size_t cap = 0; // 8-byte words of each
+    HostBuffer() = default;
+    HostBuffer(const HostBuffer &) = delete;
+    HostBuffer &operator=(const HostBuffer &) = delete;
+    ~HostBuffer() { release(); }
+    void reserve(size_t words);
+    void release();
 };
 
 class Potential {
@@ -93,6 +108,9 @@ class Potential {
     // Reads device status flags (synchronises the stream) and raises the
     // reference's error message for a bad box.
     virtual void check_device_status(hipStream_t stream) {}
+    // The device words that check_device_status() reads (non-zero: it raises).
+    virtual void status_words(std::vector<const int *> &out) const {}
+    HostBuffer host_buffer;
 
     virtual void du_dp_fixed_to_float(int N, int P, const uint64_t *du_dp, double *out) const;
 
@@ -158,6 +176,7 @@ class NonbondedAllPairs : public Potential {
                              uint64_t *dg, uint64_t *d_hl, hipStream_t stream) override;
     void validate_host(int N, int P, const double *h_box) const override;
     void check_device_status(hipStream_t stream) override;
+    void status_words(std::vector<const int *> &out) const override;
     void du_dp_fixed_to_float(int N, int P, const uint64_t *du_dp, double *out) const override;
 
     void set_nblist_padding(double padding);
@@ -283,6 +302,7 @@ class SummedPotential : public Potential {
                             uint64_t *d_hl, hipStream_t stream) override;
     void validate_host(int N, int P, const double *h_box) const override;
     void check_device_status(hipStream_t stream) override;
+    void status_words(std::vector<const int *> &out) const override;
     void du_dp_fixed_to_float(int N, int P, const uint64_t *du_dp, double *out) const override;
     std::vector<PotentialPtr> pots_;
     std::vector<int> sizes_;
@@ -303,6 +323,7 @@ class FanoutSummedPotential : public Potential {
                             uint64_t *d_hl, hipStream_t stream) override;
     void validate_host(int N, int P, const double *h_box) const override;
     void check_device_status(hipStream_t stream) override;
+    void status_words(std::vector<const int *> &out) const override;
     void du_dp_fixed_to_float(int N, int P, const uint64_t *du_dp, double *out) const override;
     std::vector<PotentialPtr> pots_;
 
