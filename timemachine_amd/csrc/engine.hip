@@ -1086,6 +1086,7 @@ Engine::Engine(const std::vector<SystemSpec> &systems) : impl_(new Impl) {
             std::copy(nb->offset_.begin(), nb->offset_.end(), offset.begin() + I.atom0[s]);
         }
         st.nb_margin = NB_LIST_MARGIN;
+        st.map_atoms = true;
         st.init(ys, subset);
         h_params = params;
         upload_vec(d_params, params);

@@ -151,7 +151,9 @@ struct NbState {
     // [total_blocks * NB_MAX_PIECES] (empty for views: one piece)
     DeviceArray<uint32_t> piece_buf;
     DeviceArray<int> piece_cnt;
-    DeviceArray<int> slot_of; // [sum n_atoms] sorted slot of each global atom, -1: none (empty for views)
+    bool map_atoms = false;   // set before init(): slot_of is kept
+    DeviceArray<int> slot_of; // [sum n_atoms] sorted slot of each global atom, -1: none
+    DeviceArray<uint64_t> cleared; // what red_slots, sorted_acc and order_done point into, cleared at once
     // [6 * total_slots] the tiles' sums of force and parameter derivatives by slot,
     // zero between launches (empty for views: tiles add to the atoms)
     DeviceArray<uint64_t> sorted_acc;

@@ -1114,7 +1114,6 @@ void NbState::init(const std::vector<NbSys> &sys_in, const std::vector<int> &sub
     status.alloc(S);
     tile_count.alloc(static_cast<size_t>(S) * NB_TILE_LANES);
     tile_prefix.alloc(S + 1);
-    order_done.alloc(1);
     tile_row.alloc(total_tiles);
     tile_order.alloc(total_tiles);
     tile_atoms.alloc(static_cast<size_t>(total_tiles) * TILE);
@@ -1135,18 +1134,22 @@ void NbState::init(const std::vector<NbSys> &sys_in, const std::vector<int> &sub
     bb_ext.alloc(total_blocks);
     piece_buf.alloc(static_cast<size_t>(total_blocks) * NB_MAX_PIECES * TILE);
     piece_cnt.alloc(static_cast<size_t>(total_blocks) * NB_MAX_PIECES);
-    slot_of.alloc(std::max(total_atoms_end, 1));
-    launch_fill_i32(slot_of.ptr, slot_of.n, -1, 0);
-    sorted_acc.alloc(static_cast<size_t>(total_slots) * 6);
-    red_slots.alloc(static_cast<size_t>(S) * NB_RED_SLOTS);
+    if (map_atoms) {
+        slot_of.alloc(std::max(total_atoms_end, 1));
+        launch_fill_i32(slot_of.ptr, slot_of.n, -1, 0);
+    }
+    const size_t n_red = static_cast<size_t>(S) * NB_RED_SLOTS, n_sorted = static_cast<size_t>(total_slots) * 6;
+    const size_t red_words = n_red * sizeof(NbRedSlot) / sizeof(uint64_t);
+    cleared.alloc(red_words + n_sorted + 1);
+    red_slots.view(reinterpret_cast<NbRedSlot *>(cleared.ptr), n_red);
+    sorted_acc.view(cleared.ptr + red_words, n_sorted);
+    order_done.view(reinterpret_cast<int *>(cleared.ptr + red_words + n_sorted), 1);
     nblist_x.alloc(static_cast<size_t>(total_atoms_end) * 3);
     nblist_box.alloc(static_cast<size_t>(S) * 9);
     status.zero();
     tile_count.zero();
     tile_prefix.zero();
-    order_done.zero();
-    sorted_acc.zero();
-    red_slots.zero();
+    cleared.zero();
     nblist_x.zero();
     nblist_box.zero();
     launch_fill_i32(rebuild.ptr, S, 1, 0);
