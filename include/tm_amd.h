@@ -13,7 +13,9 @@
  *     potential defines them; uint64 outputs are 64-bit fixed point
  *     (2^36 for du_dx, u, du_dl; nonbonded du_dp uses 2^36 / 2^37 / 2^38 for
  *     charge / sigma / epsilon columns) and accumulate into caller-zeroed buffers;
- *   - a NULL output pointer means "not requested".
+ *   - a NULL output pointer means "not requested";
+ *   - several threads may call into one potential, or into sums that share a part:
+ *     the calls take turns, each a whole sequence of launches.
  * The library owns no global state besides the HIP device context.
  */
 #ifndef TM_AMD_H

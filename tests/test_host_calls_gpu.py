@@ -1,6 +1,6 @@
-"""Host calls share one kept buffer per potential: calls of any size and choice of
-outputs after each other, after an error, and from two threads at once give what a
-fresh potential gives."""
+"""Calls share what a potential keeps (host buffer, neighborlist, tile sums): calls of
+any size and choice of outputs after each other, after an error, and from two threads
+at once give what a fresh potential gives."""
 
 import threading
 
@@ -35,17 +35,54 @@ def test_calls_after_each_other_and_from_threads(gpu, n, others):
             np.testing.assert_array_equal(g, e)
     only = pot.execute_selective(*cases[0], 0.3, False, False, False, True)
     assert only[0] is None and only[3] == pot.execute(*cases[0], 0.3)[3]
+    _in_threads([lambda k=k: pot.execute_fixed_raw(*cases[k], 0.3) for k in range(2)], want[:2])
+
+
+def _in_threads(calls, want, repeats=20):
+    """Every call in a thread of its own, over and over: each result is its own."""
     failed = []
 
-    def work(k):
-        for _ in range(20):
-            got = pot.execute_fixed_raw(*cases[k], 0.3)
-            failed.extend(1 for g, e in zip(got, want[k]) if not np.array_equal(g, e))
+    def work(call, expect):
+        for _ in range(repeats):
+            failed.extend(1 for g, e in zip(call(), expect) if not np.array_equal(g, e))
 
-    threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    threads = [threading.Thread(target=work, args=a) for a in zip(calls, want)]
     [t.start() for t in threads]
     [t.join() for t in threads]
     assert not failed
+
+
+def _charges(rng, n, interpolated):
+    g = int(np.ceil(n ** (1 / 3)))
+    sites = np.stack(np.meshgrid(*[np.arange(g)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
+    x = (sites + rng.uniform(0.2, 0.8, (n, 3))) * (3.0 / g)
+    p = np.stack([rng.normal(size=n), np.full(n, 0.1), rng.uniform(0.3, 0.9, n)], 1)
+    return x, np.concatenate([p, 0.9 * p]) if interpolated else p, np.eye(3) * 3.0
+
+
+@pytest.mark.parametrize("interpolated", [False, True])
+@pytest.mark.parametrize("n,same", [(700, True), (700, False)])
+def test_threads_in_one_nonbonded_potential(gpu, n, same, interpolated):
+    """The neighborlist and the tiles' sums belong to the potential: calls from two
+    threads use them one after the other, alone or as a part that two sums share."""
+    rng = np.random.default_rng(n + same)
+    plane, offset = np.zeros(n, np.int32), (rng.random(n) < 0.05).astype(np.int32)
+    kind = custom_ops.NonbondedAllPairs_f32_interpolated if interpolated else custom_ops.NonbondedAllPairs_f32
+
+    def new():
+        return kind(None, plane, offset, 2.0, 1.2)
+
+    a = _charges(rng, n, interpolated)
+    b = a if same else _charges(rng, n, interpolated)
+    want = [new().execute_fixed_raw(*c, 0.4) for c in (a, b)]
+    pot = new()
+    _in_threads([lambda c=c: pot.execute_fixed_raw(*c, 0.4) for c in (a, b)], want)
+    sums = [custom_ops.SummedPotential([pot], [a[1].size]), custom_ops.FanoutSummedPotential([pot])]
+    _in_threads([lambda c=c, s=s: s.execute_fixed_raw(*c, 0.4) for c, s in zip((a, b), sums)], want)
+    frames = np.stack([b[0]] * 2), b[1][None], np.stack([b[2]] * 2), np.array([0.4, 0.7]), True, True, True, True
+    want_batch = new().execute_selective_batch(*frames)
+    _in_threads([lambda: pot.execute_fixed_raw(*a, 0.4), lambda: pot.execute_selective_batch(*frames)],
+                [want[0], want_batch], 8)
 
 
 def test_call_after_an_error(gpu):

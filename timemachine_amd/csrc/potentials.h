@@ -31,9 +31,9 @@ enum class PotKind {
 };
 
 // Device workspace and pinned staging of a potential's host calls, kept between
-// calls and freed with the potential. As large as its largest call.
+// calls and freed with the potential. As large as its largest call; used by one
+// call at a time (PotentialCall).
 struct HostBuffer {
-    std::mutex m;
     uint64_t *dev = nullptr, *pin = nullptr;
     size_t cap = 0; // 8-byte words of each
     HostBuffer() = default;
@@ -112,6 +112,13 @@ class Potential {
     virtual void status_words(std::vector<const int *> &out) const {}
     HostBuffer host_buffer;
 
+    // This potential and every potential it is made of.
+    virtual void parts(std::vector<Potential *> &out) { out.push_back(this); }
+    // Whether a call uses device memory kept with the potential besides
+    // host_buffer (neighborlist, sums in sorted order, temporaries).
+    virtual bool keeps_device_state() const { return false; }
+    std::mutex call_mutex; // held by the call that uses that memory (PotentialCall)
+
     virtual void du_dp_fixed_to_float(int N, int P, const uint64_t *du_dp, double *out) const;
 
     void execute_host(
@@ -143,6 +150,20 @@ class Potential {
 };
 
 using PotentialPtr = std::shared_ptr<Potential>;
+
+// Reserves what a call of p uses beyond its arguments, until the end of the
+// scope: the device state of p and of its parts (parts of a sum may belong to
+// other sums too) and, for a call with host arrays, p's host buffer. A call is a
+// sequence of launches over that memory (neighborlist, tile sums, their move to
+// the atoms), so a second thread waits for the whole sequence: launches of two
+// calls in between each other would give one the other's sums.
+class PotentialCall {
+  public:
+    PotentialCall(Potential &p, bool host);
+
+  private:
+    std::vector<std::unique_lock<std::mutex>> locks_;
+};
 
 // Hessian-vector product (execute_hvp_device) of potentials that share the
 // interpolated parameters d_p [2N, 3]: p(lambda) and its tangent once, the
@@ -177,6 +198,7 @@ class NonbondedAllPairs : public Potential {
     void validate_host(int N, int P, const double *h_box) const override;
     void check_device_status(hipStream_t stream) override;
     void status_words(std::vector<const int *> &out) const override;
+    bool keeps_device_state() const override { return true; }
     void du_dp_fixed_to_float(int N, int P, const uint64_t *du_dp, double *out) const override;
 
     void set_nblist_padding(double padding);
@@ -249,6 +271,7 @@ class NonbondedPairList : public Potential {
     void hvp_at_interpolated(int N, const double *d_x, const double *p_lam, const double *d_box, double lambda,
                              const double *d_vx, const double *vp_lam, double vl, uint64_t *d_hx, uint64_t *g,
                              uint64_t *dg, uint64_t *d_hl, hipStream_t stream) override;
+    bool keeps_device_state() const override { return interp_; }
     void du_dp_fixed_to_float(int N, int P, const uint64_t *du_dp, double *out) const override;
 
     int N_, M_;
@@ -303,6 +326,7 @@ class SummedPotential : public Potential {
     void validate_host(int N, int P, const double *h_box) const override;
     void check_device_status(hipStream_t stream) override;
     void status_words(std::vector<const int *> &out) const override;
+    void parts(std::vector<Potential *> &out) override;
     void du_dp_fixed_to_float(int N, int P, const uint64_t *du_dp, double *out) const override;
     std::vector<PotentialPtr> pots_;
     std::vector<int> sizes_;
@@ -324,6 +348,8 @@ class FanoutSummedPotential : public Potential {
     void validate_host(int N, int P, const double *h_box) const override;
     void check_device_status(hipStream_t stream) override;
     void status_words(std::vector<const int *> &out) const override;
+    void parts(std::vector<Potential *> &out) override;
+    bool keeps_device_state() const override; // hvp_tmp_
     void du_dp_fixed_to_float(int N, int P, const uint64_t *du_dp, double *out) const override;
     std::vector<PotentialPtr> pots_;
 

@@ -1,6 +1,8 @@
 // Host-side potential classes (see potentials.h).
+#include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <functional>
 #include <numeric>
 #include <set>
 
@@ -21,6 +23,24 @@ static HvpTangent hvp_tangent(const double *vx, const double *vp, double vl) {
 void Potential::du_dp_fixed_to_float(int N, int P, const uint64_t *du_dp, double *out) const {
     for (int i = 0; i < P; i++) {
         out[i] = fixed_to_double(du_dp[i], FIXED_SCALE);
+    }
+}
+
+PotentialCall::PotentialCall(Potential &p, bool host) {
+    std::vector<Potential *> all;
+    p.parts(all);
+    std::vector<Potential *> held;
+    for (Potential *q : all) {
+        if (q->keeps_device_state() || (host && q == &p)) {
+            held.push_back(q);
+        }
+    }
+    // in address order, each once: two sums over the same potentials cannot wait for each other
+    std::sort(held.begin(), held.end(), std::less<Potential *>());
+    held.erase(std::unique(held.begin(), held.end()), held.end());
+    locks_.reserve(held.size());
+    for (Potential *q : held) {
+        locks_.emplace_back(q->call_mutex);
     }
 }
 
@@ -54,13 +74,11 @@ namespace {
 // pageable memory spent more on that than on the kernels: the bonded terms of one
 // molecule 158 -> 55 us, of a 6k-atom box 207 -> 105 us, u and du/dl of 1k atoms
 // 176 -> 108 us, forces of 6k atoms 183 -> 147 us, a Hessian-vector product at 6k
-// atoms 410 -> 307 us. A second thread in the same potential meanwhile uses a
-// buffer of its own for the call.
+// atoms 410 -> 307 us.
 class HostCall {
   public:
-    HostCall(HostBuffer &kept, size_t in_words, size_t out_words)
-        : lock_(kept.m, std::try_to_lock), b_(lock_.owns_lock() ? kept : own_), in_(in_words), out_(out_words),
-          out_at_(in_words) {
+    HostCall(Potential &p, size_t in_words, size_t out_words)
+        : hold_(p, true), p_(p), b_(p.host_buffer), in_(in_words), out_(out_words), out_at_(in_words) {
         b_.reserve(in_ + out_ + STATUS_WORDS);
     }
     // the next input: n words, to be written by the caller before start(); its device address
@@ -92,9 +110,9 @@ class HostCall {
         launch_fill_u64(b_.dev + in_, out_, 0, 0);
     }
     // Waits for the outputs; raises what check_device_status() raises.
-    void finish(Potential &p) {
+    void finish() {
         std::vector<const int *> words;
-        p.status_words(words);
+        p_.status_words(words);
         int *status = reinterpret_cast<int *>(b_.pin + in_ + out_);
         const bool staged = words.size() <= 2 * STATUS_WORDS;
         {
@@ -112,7 +130,7 @@ class HostCall {
             bad = bad || status[i] != 0;
         }
         if (bad) {
-            p.check_device_status(0);
+            p_.check_device_status(0);
         }
     }
     // an output on the host, after finish()
@@ -125,8 +143,8 @@ class HostCall {
 
   private:
     static constexpr size_t STATUS_WORDS = 8;
-    HostBuffer own_;
-    std::unique_lock<std::mutex> lock_;
+    PotentialCall hold_;
+    Potential &p_;
     HostBuffer &b_;
     size_t in_, out_, in_at_ = 0, out_at_;
 };
@@ -137,7 +155,7 @@ void Potential::execute_host(int N, int P, const double *h_x, const double *h_p,
                              uint64_t *h_du_dx, uint64_t *h_du_dp, uint64_t *h_du_dl, uint64_t *h_u) {
     validate_host(N, P, h_box);
     const size_t n3 = static_cast<size_t>(N) * 3, n1 = std::max(N, 1), p1 = std::max(P, 1);
-    HostCall call(host_buffer, n3 + 9 + std::max(P, 0),
+    HostCall call(*this, n3 + 9 + std::max(P, 0),
                   (h_du_dx ? n3 : 0) + (h_du_dp ? p1 : 0) + (h_du_dl ? n1 : 0) + (h_u ? n1 : 0));
     const double *x = call.input(h_x, n3), *box = call.input(h_box, 9);
     const double *p = P > 0 ? call.input(h_p, P) : nullptr;
@@ -145,7 +163,7 @@ void Potential::execute_host(int N, int P, const double *h_x, const double *h_p,
     uint64_t *du_dl = h_du_dl ? call.output(n1) : nullptr, *u = h_u ? call.output(n1) : nullptr;
     call.start();
     execute_device(N, P, x, p, box, lambda, du_dx, du_dp, du_dl, u, 0);
-    call.finish(*this);
+    call.finish();
     if (h_du_dx) {
         call.fetch(du_dx, h_du_dx, n3);
     }
@@ -163,6 +181,7 @@ void Potential::execute_host(int N, int P, const double *h_x, const double *h_p,
 void Potential::execute_dl_dp_host(int N, int P, const double *h_x, const double *h_p, const double *h_box,
                                    double lambda, uint64_t *h_dl_dp) {
     validate_host(N, P, h_box);
+    PotentialCall hold(*this, true);
     DeviceArray<double> x(static_cast<size_t>(N) * 3), box(9), p(std::max(P, 1));
     x.upload(h_x, static_cast<size_t>(N) * 3);
     box.upload(h_box, 9);
@@ -235,7 +254,7 @@ void Potential::execute_hvp_host(int N, int P, const double *h_x, const double *
     const double scale = std::ldexp(1.0, -e);
     const size_t np = std::max(P, 0), p1 = std::max(P, 1);
     const bool has_vp = h_vp && P > 0;
-    HostCall call(host_buffer, n3 + 9 + np + (h_vx ? n3 : 0) + (has_vp ? np : 0),
+    HostCall call(*this, n3 + 9 + np + (h_vx ? n3 : 0) + (has_vp ? np : 0),
                   (h_hx ? n3 : 0) + (h_hp ? p1 : 0) + (h_hl ? 1 : 0));
     const double *x = call.input(h_x, n3), *box = call.input(h_box, 9);
     const double *p = P > 0 ? call.input(h_p, np) : nullptr;
@@ -252,7 +271,7 @@ void Potential::execute_hvp_host(int N, int P, const double *h_x, const double *
     uint64_t *hl = h_hl ? call.output(1) : nullptr;
     call.start();
     execute_hvp_device(N, P, x, p, box, lambda, vx, vp, vl * scale, hx, hp, hl, 0);
-    call.finish(*this);
+    call.finish();
     if (h_hx) {
         const uint64_t *fixed = call.host(hx);
         for (size_t i = 0; i < n3; i++) {
@@ -276,6 +295,7 @@ void Potential::execute_batch_host(int coord_batch_size, int N, int param_batch_
     for (int i = 0; i < coord_batch_size; i++) {
         validate_host(N, P, h_box + i * 9);
     }
+    PotentialCall hold(*this, true);
     const size_t total = static_cast<size_t>(coord_batch_size) * param_batch_size * lambda_batch_size;
     DeviceArray<double> x(static_cast<size_t>(coord_batch_size) * N * 3), box(static_cast<size_t>(coord_batch_size) * 9);
     DeviceArray<double> p(std::max<size_t>(static_cast<size_t>(param_batch_size) * P, 1));
@@ -370,11 +390,13 @@ NonbondedAllPairs::NonbondedAllPairs(const std::vector<int> &plane, const std::v
 }
 
 void NonbondedAllPairs::set_nblist_padding(double padding) {
+    std::lock_guard<std::mutex> hold(call_mutex);
     padding_ = padding;
     dirty_ = true;
 }
 
 void NonbondedAllPairs::disable_hilbert_sort() {
+    std::lock_guard<std::mutex> hold(call_mutex);
     sorted_ = false;
     dirty_ = true;
 }
@@ -543,6 +565,7 @@ void NonbondedAllPairs::check_device_status(hipStream_t stream) {
 }
 
 int NonbondedAllPairs::num_tiles(hipStream_t stream) {
+    std::lock_guard<std::mutex> hold(call_mutex);
     ensure_state();
     int n = 0;
     TM_HIP_CHECK(hipMemcpyAsync(&n, st_.tile_prefix.ptr + 1, sizeof(int), hipMemcpyDeviceToHost, stream));
@@ -879,6 +902,13 @@ void SummedPotential::status_words(std::vector<const int *> &out) const {
     }
 }
 
+void SummedPotential::parts(std::vector<Potential *> &out) {
+    out.push_back(this);
+    for (auto &p : pots_) {
+        p->parts(out);
+    }
+}
+
 void SummedPotential::check_device_status(hipStream_t stream) {
     for (auto &p : pots_) {
         p->check_device_status(stream);
@@ -947,6 +977,17 @@ void FanoutSummedPotential::status_words(std::vector<const int *> &out) const {
     }
 }
 
+void FanoutSummedPotential::parts(std::vector<Potential *> &out) {
+    out.push_back(this);
+    for (auto &p : pots_) {
+        p->parts(out);
+    }
+}
+
+bool FanoutSummedPotential::keeps_device_state() const {
+    return std::any_of(pots_.begin(), pots_.end(), [](const PotentialPtr &p) { return p->interpolated_nonbonded(); });
+}
+
 void FanoutSummedPotential::check_device_status(hipStream_t stream) {
     for (auto &p : pots_) {
         p->check_device_status(stream);
@@ -993,12 +1034,12 @@ void BoundPotential::execute_host(int N, const double *h_x, const double *h_box,
                                   uint64_t *h_du_dl, uint64_t *h_u) {
     potential->validate_host(N, size(), h_box);
     const size_t n3 = static_cast<size_t>(N) * 3, n1 = std::max(N, 1);
-    HostCall call(potential->host_buffer, n3 + 9, n3 + 2 * n1);
+    HostCall call(*potential, n3 + 9, n3 + 2 * n1);
     const double *x = call.input(h_x, n3), *box = call.input(h_box, 9);
     uint64_t *du_dx = call.output(n3), *du_dl = call.output(n1), *u = call.output(n1);
     call.start();
     execute_device(N, x, box, lambda, du_dx, nullptr, du_dl, u, 0);
-    call.finish(*potential);
+    call.finish();
     call.fetch(du_dx, h_du_dx, n3);
     call.fetch(du_dl, h_du_dl, N);
     call.fetch(u, h_u, N);
