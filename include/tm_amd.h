@@ -15,7 +15,10 @@
  *     charge / sigma / epsilon columns) and accumulate into caller-zeroed buffers;
  *   - a NULL output pointer means "not requested";
  *   - several threads may call into one potential, or into sums that share a part:
- *     the calls take turns, each a whole sequence of launches.
+ *     the calls take turns, each a whole sequence of launches. Calls with device pointers may
+ *     use different streams; each waits on its stream for the call before. Only a call that is
+ *     captured into a graph does not: the caller orders the graph's launches with other calls
+ *     into the potential.
  * The library owns no global state besides the HIP device context.
  */
 #ifndef TM_AMD_H

@@ -1,0 +1,90 @@
+"""Device-pointer calls of one potential on several streams, between host calls and
+captured into a graph: each call's outputs are those of a fresh potential."""
+
+import numpy as np
+import pytest
+import torch
+
+from timemachine_amd import _lib
+from timemachine_amd.lib import custom_ops
+
+pytestmark = pytest.mark.gpu
+
+LAM = 0.4
+
+
+def _system(rng, n):
+    g = int(np.ceil(n ** (1 / 3)))
+    sites = np.stack(np.meshgrid(*[np.arange(g)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
+    x = (sites + rng.uniform(0.2, 0.8, (n, 3))) * (3.0 / g)
+    return x, np.stack([rng.normal(size=n), np.full(n, 0.1), rng.uniform(0.3, 0.9, n)], 1), np.eye(3) * 3.0
+
+
+class _Call:
+    """One configuration's device inputs and outputs."""
+
+    def __init__(self, x, p, box):
+        self.n = len(x)
+        self.ins = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (x, p, box)]
+        self.outs = [torch.zeros(k * self.n, dtype=torch.int64, device="cuda") for k in (3, 3, 1, 1)]
+
+    def launch(self, pot, stream):
+        for o in self.outs:
+            o.zero_()
+        _lib.call("tm_potential_execute_device", pot.handle, self.n, self.n * 3, *[a.data_ptr() for a in self.ins], LAM,
+                  *[o.data_ptr() for o in self.outs], stream.cuda_stream)
+
+    def get(self):
+        return [o.cpu().numpy().view(np.uint64) for o in self.outs]
+
+
+def _setup(n, same):
+    rng = np.random.default_rng(n)
+    plane, offset = np.zeros(n, np.int32), (rng.random(n) < 0.05).astype(np.int32)
+    configs = [_system(rng, n)]
+    configs.append(configs[0] if same else _system(rng, n))
+    new = lambda: custom_ops.NonbondedAllPairs_f32(None, plane, offset, 2.0, 1.2)
+    return new, configs, [new().execute_fixed_raw(*c, LAM) for c in configs]
+
+
+def _check(got, want):
+    for g, w in zip(got, want):
+        np.testing.assert_array_equal(g, w)
+
+
+@pytest.mark.parametrize("n,same", [(700, True), (700, False), (4000, False)])
+def test_two_streams(gpu, n, same):
+    new, configs, want = _setup(n, same)
+    pot = new()
+    calls, streams = [_Call(*c) for c in configs], [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for rep in range(10):
+        for c, s in zip(calls, streams):
+            with torch.cuda.stream(s):
+                c.launch(pot, s)
+        if rep % 3 == 2:  # a host call while both may be in flight
+            _check(pot.execute_fixed_raw(*configs[rep % 2], LAM), want[rep % 2])
+        torch.cuda.synchronize()
+        for c, w in zip(calls, want):
+            _check(c.get(), w)
+
+
+def test_captured_call(gpu):
+    new, configs, want = _setup(700, False)
+    pot = new()
+    calls, stream = [_Call(*c) for c in configs], torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        calls[1].launch(pot, stream)  # the potential's arrays exist before the capture
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        calls[0].launch(pot, stream)
+    for _ in range(4):
+        graph.replay()
+        torch.cuda.synchronize()
+        _check(calls[0].get(), want[0])
+        with torch.cuda.stream(stream):
+            calls[1].launch(pot, stream)
+        torch.cuda.synchronize()
+        _check(calls[1].get(), want[1])

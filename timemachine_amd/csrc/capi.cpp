@@ -304,7 +304,7 @@ int tm_potential_execute_device(tm_potential *p, int N, int P, const double *d_x
                                 const double *d_box, double lambda, uint64_t *d_du_dx, uint64_t *d_du_dp,
                                 uint64_t *d_du_dl, uint64_t *d_u, void *stream) {
     return guarded([&] {
-        PotentialCall hold(*p->p, false);
+        PotentialCall hold(*p->p, static_cast<hipStream_t>(stream), false);
         p->p->execute_device(N, P, d_x, d_p, d_box, lambda, d_du_dx, d_du_dp, d_du_dl, d_u,
                              static_cast<hipStream_t>(stream));
     });
@@ -341,7 +341,7 @@ int tm_potential_execute_dl_dp_device(tm_potential *p, int N, int P, const doubl
         if (!d_dl_dp) {
             throw Error("execute_dl_dp: output buffer is null");
         }
-        PotentialCall hold(*p->p, false);
+        PotentialCall hold(*p->p, static_cast<hipStream_t>(stream), false);
         p->p->execute_dl_dp_device(N, P, d_x, d_p, d_box, lambda, d_dl_dp, static_cast<hipStream_t>(stream));
     });
 }
@@ -360,7 +360,7 @@ int tm_potential_execute_hvp_device(tm_potential *p, int N, int P, const double 
                                     const double *d_box, double lambda, const double *d_vx, const double *d_vp,
                                     double vl, uint64_t *d_hx, uint64_t *d_hp, uint64_t *d_hl, void *stream) {
     return guarded([&] {
-        PotentialCall hold(*p->p, false);
+        PotentialCall hold(*p->p, static_cast<hipStream_t>(stream), false);
         p->p->execute_hvp_device(N, P, d_x, d_p, d_box, lambda, d_vx, d_vp, vl, d_hx, d_hp, d_hl,
                                  static_cast<hipStream_t>(stream));
     });

@@ -44,6 +44,17 @@ struct HostBuffer {
     void release();
 };
 
+// Who uses the memory that a potential keeps (PotentialCall).
+struct CallState {
+    std::mutex m;              // held by the call in progress
+    hipEvent_t done = nullptr; // after the launches of the last call that did not wait for them
+    bool pending = false;      // done was recorded
+    CallState() = default;
+    CallState(const CallState &) = delete;
+    CallState &operator=(const CallState &) = delete;
+    ~CallState();
+};
+
 class Potential {
   public:
     virtual ~Potential() = default;
@@ -117,7 +128,7 @@ class Potential {
     // Whether a call uses device memory kept with the potential besides
     // host_buffer (neighborlist, sums in sorted order, temporaries).
     virtual bool keeps_device_state() const { return false; }
-    std::mutex call_mutex; // held by the call that uses that memory (PotentialCall)
+    CallState call_state;
 
     virtual void du_dp_fixed_to_float(int N, int P, const uint64_t *du_dp, double *out) const;
 
@@ -156,13 +167,24 @@ using PotentialPtr = std::shared_ptr<Potential>;
 // other sums too) and, for a call with host arrays, p's host buffer. A call is a
 // sequence of launches over that memory (neighborlist, tile sums, their move to
 // the atoms), so a second thread waits for the whole sequence: launches of two
-// calls in between each other would give one the other's sums.
+// calls in between each other would give one the other's sums. So would launches
+// on two streams, so a call's stream first waits for the launches of the call
+// before (an event; nothing waits on the host). A call that is being captured
+// neither waits nor leaves an event: its stream orders it within the graph, and
+// whoever launches the graph orders that with other calls.
 class PotentialCall {
   public:
-    PotentialCall(Potential &p, bool host);
+    PotentialCall(Potential &p, hipStream_t stream, bool host);
+    ~PotentialCall();
+    PotentialCall(const PotentialCall &) = delete;
+    PotentialCall &operator=(const PotentialCall &) = delete;
+    void synchronised() { synchronised_ = true; } // the stream was waited for after the last launch
 
   private:
+    std::vector<Potential *> held_;
     std::vector<std::unique_lock<std::mutex>> locks_;
+    hipStream_t stream_;
+    bool captured_ = false, synchronised_ = false;
 };
 
 // Hessian-vector product (execute_hvp_device) of potentials that share the

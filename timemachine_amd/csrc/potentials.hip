@@ -26,21 +26,64 @@ void Potential::du_dp_fixed_to_float(int N, int P, const uint64_t *du_dp, double
     }
 }
 
-PotentialCall::PotentialCall(Potential &p, bool host) {
+CallState::~CallState() {
+    if (done) {
+        (void)hipEventDestroy(done);
+    }
+}
+
+PotentialCall::PotentialCall(Potential &p, hipStream_t stream, bool host) : stream_(stream) {
     std::vector<Potential *> all;
     p.parts(all);
-    std::vector<Potential *> held;
     for (Potential *q : all) {
         if (q->keeps_device_state() || (host && q == &p)) {
-            held.push_back(q);
+            held_.push_back(q);
         }
     }
     // in address order, each once: two sums over the same potentials cannot wait for each other
-    std::sort(held.begin(), held.end(), std::less<Potential *>());
-    held.erase(std::unique(held.begin(), held.end()), held.end());
-    locks_.reserve(held.size());
-    for (Potential *q : held) {
-        locks_.emplace_back(q->call_mutex);
+    std::sort(held_.begin(), held_.end(), std::less<Potential *>());
+    held_.erase(std::unique(held_.begin(), held_.end()), held_.end());
+    locks_.reserve(held_.size());
+    for (Potential *q : held_) {
+        locks_.emplace_back(q->call_state.m);
+    }
+    if (stream && !held_.empty()) {
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        TM_HIP_CHECK(hipStreamIsCapturing(stream, &status));
+        captured_ = status != hipStreamCaptureStatusNone;
+    }
+    for (Potential *q : held_) {
+        if (q->call_state.pending && !captured_) {
+            std::unique_lock<std::recursive_mutex> lock(device_mutex(), std::defer_lock);
+            if (!stream) {
+                lock.lock(); // null stream
+            }
+            TM_HIP_CHECK(hipStreamWaitEvent(stream, q->call_state.done, 0));
+        }
+    }
+}
+
+PotentialCall::~PotentialCall() {
+    for (Potential *q : held_) {
+        CallState &c = q->call_state;
+        if (captured_) {
+            continue;
+        }
+        c.pending = false; // the stream waited for it
+        if (synchronised_ || !q->keeps_device_state()) {
+            continue;
+        }
+        std::unique_lock<std::recursive_mutex> lock(device_mutex(), std::defer_lock);
+        if (!stream_) {
+            lock.lock(); // null stream
+        }
+        if ((c.done || hipEventCreateWithFlags(&c.done, hipEventDisableTiming) == hipSuccess) &&
+            hipEventRecord(c.done, stream_) == hipSuccess) {
+            c.pending = true;
+        } else { // no event: wait for the launches here
+            (void)hipGetLastError();
+            (void)hipStreamSynchronize(stream_);
+        }
     }
 }
 
@@ -78,7 +121,7 @@ namespace {
 class HostCall {
   public:
     HostCall(Potential &p, size_t in_words, size_t out_words)
-        : hold_(p, true), p_(p), b_(p.host_buffer), in_(in_words), out_(out_words), out_at_(in_words) {
+        : hold_(p, 0, true), p_(p), b_(p.host_buffer), in_(in_words), out_(out_words), out_at_(in_words) {
         b_.reserve(in_ + out_ + STATUS_WORDS);
     }
     // the next input: n words, to be written by the caller before start(); its device address
@@ -125,6 +168,7 @@ class HostCall {
             }
         }
         TM_HIP_CHECK(hipStreamSynchronize(0));
+        hold_.synchronised();
         bool bad = !staged;
         for (size_t i = 0; staged && i < words.size(); i++) {
             bad = bad || status[i] != 0;
@@ -181,7 +225,7 @@ void Potential::execute_host(int N, int P, const double *h_x, const double *h_p,
 void Potential::execute_dl_dp_host(int N, int P, const double *h_x, const double *h_p, const double *h_box,
                                    double lambda, uint64_t *h_dl_dp) {
     validate_host(N, P, h_box);
-    PotentialCall hold(*this, true);
+    PotentialCall hold(*this, 0, true);
     DeviceArray<double> x(static_cast<size_t>(N) * 3), box(9), p(std::max(P, 1));
     x.upload(h_x, static_cast<size_t>(N) * 3);
     box.upload(h_box, 9);
@@ -194,6 +238,7 @@ void Potential::execute_dl_dp_host(int N, int P, const double *h_x, const double
     check_device_status(0);
     dl_dp.download(h_dl_dp, P);
     TM_HIP_CHECK(hipStreamSynchronize(0));
+    hold.synchronised();
 }
 
 void Potential::execute_hvp_device(int N, int P, const double *d_x, const double *d_p, const double *d_box,
@@ -295,7 +340,7 @@ void Potential::execute_batch_host(int coord_batch_size, int N, int param_batch_
     for (int i = 0; i < coord_batch_size; i++) {
         validate_host(N, P, h_box + i * 9);
     }
-    PotentialCall hold(*this, true);
+    PotentialCall hold(*this, 0, true);
     const size_t total = static_cast<size_t>(coord_batch_size) * param_batch_size * lambda_batch_size;
     DeviceArray<double> x(static_cast<size_t>(coord_batch_size) * N * 3), box(static_cast<size_t>(coord_batch_size) * 9);
     DeviceArray<double> p(std::max<size_t>(static_cast<size_t>(param_batch_size) * P, 1));
@@ -346,6 +391,7 @@ void Potential::execute_batch_host(int coord_batch_size, int N, int param_batch_
         u.download(h_u, total * N);
     }
     TM_HIP_CHECK(hipStreamSynchronize(0));
+    hold.synchronised();
 }
 
 void validate_nonbonded_box(const double *h_box, double cutoff, double padding) {
@@ -390,13 +436,13 @@ NonbondedAllPairs::NonbondedAllPairs(const std::vector<int> &plane, const std::v
 }
 
 void NonbondedAllPairs::set_nblist_padding(double padding) {
-    std::lock_guard<std::mutex> hold(call_mutex);
+    std::lock_guard<std::mutex> hold(call_state.m);
     padding_ = padding;
     dirty_ = true;
 }
 
 void NonbondedAllPairs::disable_hilbert_sort() {
-    std::lock_guard<std::mutex> hold(call_mutex);
+    std::lock_guard<std::mutex> hold(call_state.m);
     sorted_ = false;
     dirty_ = true;
 }
@@ -565,11 +611,12 @@ void NonbondedAllPairs::check_device_status(hipStream_t stream) {
 }
 
 int NonbondedAllPairs::num_tiles(hipStream_t stream) {
-    std::lock_guard<std::mutex> hold(call_mutex);
+    PotentialCall hold(*this, stream, true);
     ensure_state();
     int n = 0;
     TM_HIP_CHECK(hipMemcpyAsync(&n, st_.tile_prefix.ptr + 1, sizeof(int), hipMemcpyDeviceToHost, stream));
     TM_HIP_CHECK(hipStreamSynchronize(stream));
+    hold.synchronised();
     return n;
 }
 
