@@ -1,5 +1,6 @@
 """Device-pointer calls of one potential on several streams, between host calls and
-captured into a graph: each call's outputs are those of a fresh potential."""
+captured into a graph: each call's outputs are those of a fresh potential. The faults
+that a device call leaves in its status word are raised by the next host call."""
 
 import numpy as np
 import pytest
@@ -88,3 +89,27 @@ def test_captured_call(gpu):
             calls[1].launch(pot, stream)
         torch.cuda.synchronize()
         _check(calls[1].get(), want[1])
+
+
+@pytest.mark.parametrize("parts", [1, 17])  # 17: more status words than a host call stages
+def test_status_of_a_device_call_is_raised_by_the_next_host_call(gpu, parts):
+    """Device calls do not validate on the host. The box is found too small on the
+    device, the next host call raises what the status word says and clears it, and
+    the one after is right again."""
+    new, configs, want = _setup(700, True)
+    x, p, box = configs[0]
+    pot = new()
+    pots = [new() for _ in range(parts - 1)] + [pot]
+    total = custom_ops.SummedPotential(pots, [p.size] * parts)
+    params = np.concatenate([p] * parts)
+    first = total.execute_fixed_raw(x, params, box, LAM)
+    call, stream = _Call(x, p, np.eye(3) * 1.5), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for _ in range(2):
+        with torch.cuda.stream(stream):
+            call.launch(pot, stream)
+        with pytest.raises(RuntimeError, match="more than half of the box width"):
+            total.execute_fixed_raw(x, params, box, LAM)
+        assert not any(o.any() for o in call.get())  # nothing evaluated in that box
+        _check(total.execute_fixed_raw(x, params, box, LAM), first)
+        _check(pot.execute_fixed_raw(x, p, box, LAM), want[0])

@@ -86,14 +86,34 @@ def test_threads_in_one_nonbonded_potential(gpu, n, same, interpolated):
 
 
 def test_call_after_an_error(gpu):
+    """After a call refused on the host (box), one refused once its inputs were under
+    way (parameter count), and one of a sum refused after its first part's launches."""
     rng = np.random.default_rng(0)
     n = 200
-    x, p = rng.uniform(0, 4, (n, 3)), np.stack([rng.normal(size=n), np.full(n, 0.1), np.full(n, 0.5)], 1)
-    zero = np.zeros(n, np.int32)
-    pot = custom_ops.NonbondedAllPairs_f32(None, zero, zero, 2.0, 1.2)
-    want = custom_ops.NonbondedAllPairs_f32(None, zero, zero, 2.0, 1.2).execute_fixed_raw(x, p, np.eye(3) * 4, 0.0)
-    for _ in range(2):
-        with pytest.raises(RuntimeError):
-            pot.execute(x, p, np.eye(3) * 1.5, 0.0)
-        for g, e in zip(pot.execute_fixed_raw(x, p, np.eye(3) * 4, 0.0), want):
+    x, p, box = _charges(rng, n, False)
+    bond = _bond(n)
+    bx, bp, bbox = _inputs(rng, n)
+    pot = custom_ops.NonbondedAllPairs_f32(None, np.zeros(n, np.int32), np.zeros(n, np.int32), 2.0, 1.2)
+    both = custom_ops.SummedPotential([pot, bond], [p.size, bp.size])
+    wrong = custom_ops.SummedPotential([pot, bond], [p.size, bp.size - 1])
+    fresh = custom_ops.NonbondedAllPairs_f32(None, np.zeros(n, np.int32), np.zeros(n, np.int32), 2.0, 1.2)
+    want = fresh.execute_fixed_raw(x, p, box, 0.0)
+    want_bond = _bond(n).execute_fixed_raw(bx, bp, bbox, 0.3)
+    flat = np.concatenate([p.ravel(), bp.ravel()])
+    want_both = custom_ops.SummedPotential([fresh, _bond(n)], [p.size, bp.size]).execute_fixed_raw(x, flat, box, 0.0)
+
+    def same(got, expect):
+        for g, e in zip(got, expect):
             np.testing.assert_array_equal(g, e)
+
+    for _ in range(2):
+        with pytest.raises(RuntimeError, match="half of the box width"):
+            pot.execute(x, p, np.eye(3) * 1.5, 0.0)
+        same(pot.execute_fixed_raw(x, p, box, 0.0), want)
+        with pytest.raises(RuntimeError, match="expected P =="):
+            bond.execute(bx, bp.ravel()[:-1], bbox, 0.3)
+        same(bond.execute_fixed_raw(bx, bp, bbox, 0.3), want_bond)
+        with pytest.raises(RuntimeError, match="expected P =="):
+            wrong.execute(x, flat[:-1], box, 0.0)
+        same(both.execute_fixed_raw(x, flat, box, 0.0), want_both)
+        same(pot.execute_fixed_raw(x, p, box, 0.0), want)

@@ -111,18 +111,25 @@ void HostBuffer::reserve(size_t words) {
 namespace {
 
 // One call with host arrays on the null stream: inputs staged into pinned memory
-// and sent as one copy, outputs cleared by one kernel and fetched as one copy
-// together with the status words, one synchronisation. A call that allocated
-// and freed its arrays, cleared each with a memset and copied each from and to
-// pageable memory spent more on that than on the kernels: the bonded terms of one
-// molecule 158 -> 55 us, of a 6k-atom box 207 -> 105 us, u and du/dl of 1k atoms
-// 176 -> 108 us, forces of 6k atoms 183 -> 147 us, a Hessian-vector product at 6k
-// atoms 410 -> 307 us.
+// and sent as one copy, outputs cleared by one kernel and fetched as one copy, the
+// status words (one of each nonbonded part) after it, one synchronisation. A call
+// that allocated and freed its arrays, cleared each with a memset and copied each
+// from and to pageable memory spent more on that than on the kernels: the bonded
+// terms of one molecule 158 -> 55 us, of a 6k-atom box 207 -> 105 us, u and du/dl of
+// 1k atoms 176 -> 108 us, forces of 6k atoms 183 -> 147 us, a Hessian-vector product
+// at 6k atoms 410 -> 307 us.
 class HostCall {
   public:
     HostCall(Potential &p, size_t in_words, size_t out_words)
         : hold_(p, 0, true), p_(p), b_(p.host_buffer), in_(in_words), out_(out_words), out_at_(in_words) {
         b_.reserve(in_ + out_ + STATUS_WORDS);
+    }
+    // A call that raised between start() and finish() leaves nothing under way:
+    // the next one fills the same pinned words.
+    ~HostCall() {
+        if (started_ && !finished_ && hipStreamSynchronize(0) == hipSuccess) {
+            hold_.synchronised();
+        }
     }
     // the next input: n words, to be written by the caller before start(); its device address
     double *input(size_t n, double **host) {
@@ -146,6 +153,7 @@ class HostCall {
         return p;
     }
     void start() {
+        started_ = true;
         DeviceLock lock; // null stream
         if (in_) {
             TM_HIP_CHECK(hipMemcpyAsync(b_.dev, b_.pin, in_ * sizeof(uint64_t), hipMemcpyHostToDevice, 0));
@@ -168,6 +176,7 @@ class HostCall {
             }
         }
         TM_HIP_CHECK(hipStreamSynchronize(0));
+        finished_ = true;
         hold_.synchronised();
         bool bad = !staged;
         for (size_t i = 0; staged && i < words.size(); i++) {
@@ -191,6 +200,7 @@ class HostCall {
     Potential &p_;
     HostBuffer &b_;
     size_t in_, out_, in_at_ = 0, out_at_;
+    bool started_ = false, finished_ = false;
 };
 
 } // namespace
