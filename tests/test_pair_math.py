@@ -56,6 +56,23 @@ def test_displacements_on_the_box_grid_are_exact(pc, L):
         assert Fraction(pc.pc_frame_delta(L, xi, xj, c)) == d
 
 
+@pytest.mark.parametrize("L", [3.1, 40.0, 999.0, 2.0**20 - 1, 2.0**20, 1.7e6, 1e9, 1e12])
+def test_grid_error_stays_below_the_pair_terms(pc, L):
+    """Pairs near the origin of a box of any size: the grid moves a displacement by
+    at most 2^-52 times the power of two above L per axis, and by nothing from 2^20 nm on,
+    where that would pass 2.4e-10 nm (a relative 3e-8 of the steepest pair force at 0.1 nm,
+    the FP32 exponential of the Coulomb term has 1.2e-7)."""
+    rng = np.random.default_rng(3)
+    for _ in range(200):
+        xi = rng.uniform(-2, 2)
+        xj = xi + rng.uniform(-1.2, 1.2)
+        got = Fraction(pc.pc_delta(L, xi, xj))
+        if L < 2.0**20:
+            assert abs(got - (Fraction(xi) - Fraction(xj))) <= Fraction(2.0 ** math.ceil(math.log2(L)) * 2.0**-52)
+        else:
+            assert got == Fraction(xi - xj)
+
+
 def test_coulomb_factors(pc):
     """Force bracket and erfc against the closed forms over the fit's range
     (x up to 3): the FP32 exponential's 1.2e-7 and the fit's 2e-8. The paired

@@ -49,7 +49,9 @@ TM_HD inline double min_image_d(double d, double box, double inv_box) {
 // a pair's displacement has the same bits whatever image its atoms are held in
 // and whichever kernel forms it. Rounding to the grid moves a coordinate by at
 // most 2^-53 of that power of two (4.4e-16 nm in a 4 nm box, half an FP64 ulp
-// of a coordinate there).
+// of a coordinate there). From 2^20 nm on, where that would come near the error of
+// the pair terms (1.2e-10 nm, a relative 2e-8 of the force at 0.1 nm), coordinates
+// stay as they are and only pairs across a face lose the exactness.
 struct BoxAxis {
     double edge, inv, magic;
     TM_HD explicit BoxAxis(double L) {
@@ -58,7 +60,7 @@ struct BoxAxis {
         const uint64_t p2 = bits & 0x7FF0000000000000ull;
         double p;
         __builtin_memcpy(&p, &p2, sizeof(p));
-        const double top = p == L ? p : 2.0 * p; // the power of two at or above L
+        const double top = L < 0x1p20 ? (p == L ? p : 2.0 * p) : 0.0; // the power of two at or above L
         edge = (L + top) - top;
         inv = 1.0 / L;
         magic = 1.5 * top;
