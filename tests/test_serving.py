@@ -13,6 +13,20 @@ def test_estimate_system_bytes_grows_and_covers_tiles():
     assert b >= (nb * (nb + 1) // 2 + nb) * 64 * 4
 
 
+def _tile_capacity(k):
+    """NbState's tile slots of k atoms: the largest that the 16 counters can hand out."""
+    rows = -(-k // 64)
+    return max(j + 16 * (sum(-(-(k - 64 * r) // 64) + 1 for r in range(j, rows, 16)) - 1) + 1
+               for j in range(min(16, rows)))
+
+
+def test_estimate_system_bytes_covers_the_tile_capacity():
+    for n in [1, 63, 64, 65, 700, 1024, 1025, 1872, 6060, 6372, 27036, 36000, 131072]:
+        nb = -(-n // 64)
+        # plus 104 bytes of sorted copies and sums a slot, build pieces and the engine's state
+        assert serving.estimate_system_bytes(n) >= _tile_capacity(n) * 264 + nb * 64 * 600 + 4096
+
+
 def test_ti_estimate_trapezoid():
     lam = np.array([0.0, 0.25, 1.0])
     du_dl = np.array([[1.0, 3.0], [4.0, 4.0], [0.0, 2.0]])  # means 2, 4, 1

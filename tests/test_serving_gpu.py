@@ -1,11 +1,15 @@
 """Continuous batching (GPU): device-to-device state handover, results
 independent of the mix (bitwise), HBM budget respected."""
 
+import ctypes
+import gc
+
 import numpy as np
 import pytest
 
 from timemachine_amd import serving
 from timemachine_amd import testsystems as ts
+from timemachine_amd.fe import lambda_windows
 from timemachine_amd.lib import custom_ops
 
 pytestmark = pytest.mark.gpu
@@ -219,3 +223,30 @@ def test_batch_status_reports_bad_box_without_raising(gpu):
     g.set_raise_faults(True)
     with pytest.raises(RuntimeError, match="Cutoff with padding is more than half of the box width"):
         g.multiple_steps(5, store_du_dl_interval=5)
+
+
+def _free_bytes():
+    gc.collect()  # engines that nobody holds any more
+    rt = ctypes.CDLL("libamdhip64.so.7")  # the copy the library already loaded
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert rt.hipDeviceSynchronize() == 0 and rt.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+@pytest.mark.parametrize("n_waters,heavy,windows", [(620, 8, 128), (2000, 40, 96), (700, 60, 128), (9000, 24, 24)])
+def test_device_bytes_are_what_the_engine_takes(gpu, n_waters, heavy, windows):
+    """The engine's own account against what the device has less of, and the admission
+    estimate above it. An allocation may take up to 2 MiB more than it asks for."""
+    job = _small_job(0, n_waters, windows, 30, 0.0, heavy=heavy)
+    small = lambda_windows.build_batch(job.system, [0.0, 1.0], 1, minimize_steps=0)
+    small.multiple_steps(30, store_du_dl_interval=1)  # everything that the process keeps is loaded
+    before = _free_bytes()
+    batch = lambda_windows.build_batch(job.system, np.linspace(0, 1, windows), 1, minimize_steps=0)
+    built = before - _free_bytes()
+    own = batch.device_bytes()
+    print(f"{job.system.N} atoms: {own / windows:.0f} bytes a system, {built / windows:.0f} taken, "
+          f"estimate {serving.estimate_system_bytes(job.system.N)}", flush=True)
+    assert own <= built <= own + 100 * 2**21
+    assert own >= 0.8 * built
+    batch.multiple_steps(30, store_du_dl_interval=1)  # a deferred barostat move's arrays and the run's du/dl
+    assert own < batch.device_bytes() <= windows * serving.estimate_system_bytes(job.system.N)

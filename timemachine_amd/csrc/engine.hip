@@ -2346,14 +2346,27 @@ int Engine::total_tiles() {
 
 size_t Engine::device_bytes() const {
     const Impl &I = *impl_;
-    size_t b = I.x.bytes() * 3 + I.v.bytes() + I.du_dx.bytes() + I.cbs.bytes() * 2 + I.atom_sys.bytes();
-    if (I.has_nb) {
-        b += I.nb.tile_atoms.bytes() + I.nb.tile_row.bytes() + I.nb.pos.bytes() * 2 + I.nb.perm.bytes() * 2 +
-             I.nb.nblist_x.bytes() + I.nb_params.bytes();
+    auto bytes = [](const auto &...arrays) { return (arrays.bytes() + ... + size_t(0)); };
+    size_t b = bytes(I.x, I.v, I.x_after, I.box, I.box_after, I.cbs, I.ccs, I.ca, I.dt, I.lam, I.du_dx, I.seed, I.u_buf,
+                     I.du_dl_buf, I.step, I.atom_sys, I.d_atom0, I.d_natoms, I.red_idx, I.run_step, I.sys_status);
+    b += bytes(I.dx_trial, I.dl_trial, I.run_dl, I.run_box_frames);
+    b += I.nb.device_bytes() + bytes(I.nb_params, I.nb_params1, I.nb_plane, I.nb_offset);
+    b += I.ig.device_bytes() + bytes(I.ig_params, I.ig_params1, I.ig_plane, I.ig_offset);
+    b += bytes(I.pl_params, I.pl_params1, I.pl_plane, I.pl_offset, I.pl_cutoffs, I.pl_betas);
+    for (int k = 0; k < 2; k++) {
+        b += bytes(I.pl_pairs[k], I.pl_sys[k], I.pl_scales[k]);
     }
-    if (I.has_ig) {
-        b += I.ig.tile_atoms.bytes() + I.ig.tile_row.bytes() + I.ig.pos.bytes() * 2 + I.ig.perm.bytes() * 2 +
-             I.ig.nblist_x.bytes() + I.ig_params.bytes();
+    b += bytes(I.bt_inc_off, I.bt_inc_items, I.bt_slots);
+    for (int k = 0; k < 3; k++) {
+        b += bytes(I.bt_idx[k], I.bt_mult[k], I.bt_offset[k], I.bt_sys[k], I.bt_params[k]);
+    }
+    b += bytes(I.b_has, I.b_interval, I.b_bstep, I.b_nmol, I.b_accepted, I.b_attempted, I.b_trig, I.b_accept, I.b_seed,
+               I.b_u_before, I.b_u_after, I.b_pressure, I.b_kT, I.b_vscale, I.b_dvol, I.b_lscale, I.b_r2);
+    b += bytes(I.g_atom, I.g_mol, I.mol_sys, I.mol_count, I.atom_mol, I.centroids);
+    b += bytes(I.obs_dudp, I.obs_dldp, I.obs_dl, I.obs_sys, I.obs_n, I.obs_inv_scale, I.obs_sum_g, I.obs_sum_ag,
+               I.obs_sum_h, I.obs_sum_a, I.obs_sum_aa);
+    for (size_t k = 0; k < I.ck_x.size(); k++) {
+        b += bytes(I.ck_x[k], I.ck_v[k], I.ck_step[k]);
     }
     return b;
 }

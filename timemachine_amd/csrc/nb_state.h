@@ -173,6 +173,9 @@ struct NbState {
     static size_t view_bytes(const NbSys &y);
     void init_view(const NbSys &y, void *arena, size_t arena_bytes, hipStream_t stream);
 
+    // Device memory of an init()ed state.
+    size_t device_bytes() const;
+
     // Force a rebuild of every system on the next prepare().
     void invalidate(hipStream_t stream);
     int find_pieces() const; // waves per row block in the neighborlist build

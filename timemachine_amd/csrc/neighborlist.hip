@@ -1156,6 +1156,13 @@ void NbState::init(const std::vector<NbSys> &sys_in, const std::vector<int> &sub
     device_synchronize();
 }
 
+size_t NbState::device_bytes() const {
+    return sys.bytes() + subset.bytes() + rebuild.bytes() + status.bytes() + tile_count.bytes() + tile_prefix.bytes() +
+           tile_row.bytes() + tile_order.bytes() + tile_atoms.bytes() + perm.bytes() + keys.bytes() + pos.bytes() +
+           par.bytes() + dpar.bytes() + bb_ctr.bytes() + bb_ext.bytes() + piece_buf.bytes() + piece_cnt.bytes() +
+           slot_of.bytes() + cleared.bytes() + nblist_x.bytes() + nblist_box.bytes();
+}
+
 void NbState::invalidate(hipStream_t stream) { launch_fill_i32(rebuild.ptr, S, 1, stream); }
 
 // Waves per row block in the neighborlist build. One wave scans a row

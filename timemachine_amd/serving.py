@@ -87,12 +87,16 @@ class JobResult:
 
 
 def estimate_system_bytes(n_atoms: int) -> int:
-    """Upper bound of the device memory one system takes in the engine: per-atom
-    state and sorted copies (~400 B/atom) plus the neighborlist tile buffer
-    (capacity nb (nb + 1) / 2 + nb tiles of 64 column indices and a row)."""
+    """Upper bound of the device memory one system takes in the engine: state,
+    sorted copies, tile sums and the terms and force slots of a solvated ligand
+    (577 to 603 bytes an atom slot for 2k to 27k atoms and ligands of up to 60 heavy
+    atoms, 64 more with interpolated parameters), 264 bytes a tile of the neighborlist
+    (64 column indices, row, order) and the partial sums. The tile capacity is that
+    of 16 interleaved counters: at most nb (nb + 1) / 2 + nb for nb row blocks, plus
+    what the fullest counter's holes add, below 8 nb + 136."""
     nb = -(-n_atoms // TILE)
-    tiles = nb * (nb + 1) // 2 + nb
-    return 400 * (nb * TILE) + tiles * (TILE * 4 + 4) + 4096
+    tiles = nb * (nb + 1) // 2 + 9 * nb + 136
+    return 700 * (nb * TILE) + tiles * (TILE * 4 + 8) + 32768
 
 
 def ti_estimate(lambdas: Sequence[float], du_dl: np.ndarray) -> float:
