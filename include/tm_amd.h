@@ -76,6 +76,9 @@ int tm_nonbonded_interaction_group_create(int N, int NR, const int32_t *row_atom
 int tm_nonbonded_all_pairs_set_nblist_padding(tm_potential *p, double padding);
 /* NonbondedAllPairs::disable_hilbert_sort, nonbonded_all_pairs.cu:185-187 */
 int tm_nonbonded_all_pairs_disable_hilbert_sort(tm_potential *p);
+/* One-wave workgroups of the tile kernel in later calls, as tm_batch_set_tile_grid (results do not
+ * depend on it; for tests). */
+int tm_nonbonded_all_pairs_set_tile_grid(tm_potential *p, int grid);
 /* Tiles of the current neighborlist (no reference counterpart; diagnostics). */
 int tm_nonbonded_all_pairs_num_tiles(tm_potential *p, int *out);
 

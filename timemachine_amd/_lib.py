@@ -33,6 +33,7 @@ _SIGS = {
     "tm_nonbonded_all_pairs_interpolated_create": (c_int, [c_int, _PI, _PI, c_double, c_double, _PI, c_int, _PPV]),
     "tm_nonbonded_all_pairs_set_nblist_padding": (c_int, [_P, c_double]),
     "tm_nonbonded_all_pairs_disable_hilbert_sort": (c_int, [_P]),
+    "tm_nonbonded_all_pairs_set_tile_grid": (c_int, [_P, c_int]),
     "tm_nonbonded_all_pairs_num_tiles": (c_int, [_P, POINTER(c_int)]),
     "tm_nonbonded_pair_list_create": (
         c_int,

@@ -222,6 +222,25 @@ int tm_nonbonded_all_pairs_disable_hilbert_sort(tm_potential *p) {
     });
 }
 
+// The kernel forms wave * chunk in 32-bit integers; 2^24 workgroups keeps that
+// below 2^31 for any tile count that fits in device memory.
+static int checked_tile_grid(int grid) {
+    if (grid < 0 || grid > (1 << 24)) {
+        throw Error("tile grid must be in [0, 16777216]");
+    }
+    return grid;
+}
+
+int tm_nonbonded_all_pairs_set_tile_grid(tm_potential *p, int grid) {
+    return guarded([&] {
+        auto nb = std::dynamic_pointer_cast<NonbondedAllPairs>(p->p);
+        if (!nb) {
+            throw Error("not a NonbondedAllPairs");
+        }
+        nb->set_tile_grid(checked_tile_grid(grid));
+    });
+}
+
 int tm_nonbonded_all_pairs_num_tiles(tm_potential *p, int *out) {
     return guarded([&] {
         auto nb = std::dynamic_pointer_cast<NonbondedAllPairs>(p->p);
@@ -1093,14 +1112,7 @@ int tm_batch_total_tiles(tm_batch *b, int *out) {
 }
 
 int tm_batch_set_tile_grid(tm_batch *b, int grid) {
-    return guarded([&] {
-        // the kernel forms wave * chunk in 32-bit integers; 2^24 workgroups keeps
-        // that below 2^31 for any tile count that fits in device memory
-        if (grid < 0 || grid > (1 << 24)) {
-            throw Error("tile grid must be in [0, 16777216]");
-        }
-        b->eng->tile_grid = grid;
-    });
+    return guarded([&] { b->eng->tile_grid = checked_tile_grid(grid); });
 }
 
 int tm_batch_set_build_pieces(tm_batch *b, int pieces) {

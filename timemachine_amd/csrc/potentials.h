@@ -225,6 +225,7 @@ class NonbondedAllPairs : public Potential {
 
     void set_nblist_padding(double padding);
     void disable_hilbert_sort();
+    void set_tile_grid(int grid); // workgroups of the tile kernel, 0 = default
     // Number of tiles of the current neighborlist (synchronises).
     int num_tiles(hipStream_t stream);
     // execute_device with every intermediate array in caller-provided device
@@ -250,6 +251,7 @@ class NonbondedAllPairs : public Potential {
     void ensure_state();
     void validate_sizes(int N, int P) const;
     bool dirty_ = true;
+    int tile_grid_ = 0;
     DeviceArray<int> d_plane_, d_offset_;
     DeviceArray<uint64_t> dp_tmp_; // du/dp at the interpolated parameters [N, 3]
     InterpHvpScratch hvp_tmp_;

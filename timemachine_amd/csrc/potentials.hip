@@ -457,6 +457,11 @@ void NonbondedAllPairs::disable_hilbert_sort() {
     dirty_ = true;
 }
 
+void NonbondedAllPairs::set_tile_grid(int grid) {
+    std::lock_guard<std::mutex> hold(call_state.m);
+    tile_grid_ = grid;
+}
+
 NbSys NonbondedAllPairs::descriptor() const {
     NbSys y{};
     y.atom0 = 0;
@@ -541,10 +546,10 @@ void NonbondedAllPairs::execute_device(int N, int P, const double *d_x, const do
             dp_tmp_.alloc(static_cast<size_t>(N_) * 3);
         }
         launch_fill_u64(dp_tmp_.ptr, static_cast<size_t>(N_) * 3, 0, stream);
-        st_.compute(d_box, d_du_dx, dp_tmp_.ptr, d_du_dl, d_u, stream);
+        st_.compute(d_box, d_du_dx, dp_tmp_.ptr, d_du_dl, d_u, stream, tile_grid_);
         launch_split_interpolated_du_dp(N_, lambda, dp_tmp_.ptr, d_du_dp, stream);
     } else {
-        st_.compute(d_box, d_du_dx, d_du_dp, d_du_dl, d_u, stream);
+        st_.compute(d_box, d_du_dx, d_du_dp, d_du_dl, d_u, stream, tile_grid_);
     }
 }
 
@@ -557,7 +562,7 @@ void NonbondedAllPairs::execute_dl_dp_device(int N, int P, const double *d_x, co
     }
     st_.prepare(d_x, d_p, interp_ ? d_p + N_ * 3 : nullptr, d_box, d_plane_.ptr, d_offset_.ptr, nullptr, lambda,
                 stream);
-    st_.compute_dl_dp(d_box, d_dl_dp, stream);
+    st_.compute_dl_dp(d_box, d_dl_dp, stream, tile_grid_);
 }
 
 void NonbondedAllPairs::execute_hvp_device(int N, int P, const double *d_x, const double *d_p, const double *d_box,

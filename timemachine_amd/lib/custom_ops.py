@@ -349,6 +349,9 @@ class NonbondedAllPairs_f32(Potential):
     def disable_hilbert_sort(self):
         call("tm_nonbonded_all_pairs_disable_hilbert_sort", self._h)
 
+    def set_tile_grid(self, grid: int):
+        call("tm_nonbonded_all_pairs_set_tile_grid", self._h, int(grid))
+
     def num_tiles(self) -> int:
         n = ctypes.c_int(0)
         call("tm_nonbonded_all_pairs_num_tiles", self._h, ctypes.byref(n))
