@@ -52,14 +52,14 @@ struct SortedForces {
 void launch_atom_forces(const BondedIncidence &inc, const uint64_t *slots, const SortedForces &s0,
                         const SortedForces &s1, uint64_t *du_dx, hipStream_t stream);
 
-// All bonded terms of a batch in one launch. With slots the per-atom forces go
-// to force slots (see above) instead of du_dx.
+// All bonded terms of a batch in one launch; the per-atom forces go to force slots
+// (see above).
 struct BondedSet {
     BondedTerms t[3];   // by BondedKind
-    uint64_t *slots[3]; // or nullptr
+    uint64_t *slots[3]; // nullptr: no forces
 };
-void launch_bonded_all(const BondedSet &b, const double *x, const double *lambdas, const int *red_idx, uint64_t *du_dx,
-                       uint64_t *du_dl, uint64_t *u, hipStream_t stream);
+void launch_bonded_all(const BondedSet &b, const double *x, const double *lambdas, const int *red_idx, uint64_t *du_dl,
+                       uint64_t *u, hipStream_t stream);
 
 // dl_dp: write d(du/dlambda)/dp into du_dp (every other output must be null).
 void launch_bonded(BondedKind kind, const BondedTerms &t, const double *x, const double *lambdas, double lambda0,

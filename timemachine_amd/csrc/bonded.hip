@@ -205,17 +205,16 @@ __global__ __launch_bounds__(TERM_BLOCK) void k_bonded_all(const BondedSet b, co
                                                            const double *__restrict__ x,
                                                            const double *__restrict__ lambdas,
                                                            const int *__restrict__ red_idx,
-                                                           uint64_t *__restrict__ du_dx, uint64_t *__restrict__ du_dl,
-                                                           uint64_t *__restrict__ u) {
+                                                           uint64_t *__restrict__ du_dl, uint64_t *__restrict__ u) {
     const int g = blockIdx.x;
     if (g < g1) {
-        bonded_term<BondedKind::Bond>(b.t[0], g * TERM_BLOCK + threadIdx.x, x, lambdas, 0.0, red_idx, du_dx, nullptr,
-                                      du_dl, u, 0, b.slots[0]);
+        bonded_term<BondedKind::Bond>(b.t[0], g * TERM_BLOCK + threadIdx.x, x, lambdas, 0.0, red_idx, nullptr,
+                                      nullptr, du_dl, u, 0, b.slots[0]);
     } else if (g < g2) {
-        bonded_term<BondedKind::Angle>(b.t[1], (g - g1) * TERM_BLOCK + threadIdx.x, x, lambdas, 0.0, red_idx, du_dx,
+        bonded_term<BondedKind::Angle>(b.t[1], (g - g1) * TERM_BLOCK + threadIdx.x, x, lambdas, 0.0, red_idx, nullptr,
                                        nullptr, du_dl, u, 0, b.slots[1]);
     } else {
-        bonded_term<BondedKind::Torsion>(b.t[2], (g - g2) * TERM_BLOCK + threadIdx.x, x, lambdas, 0.0, red_idx, du_dx,
+        bonded_term<BondedKind::Torsion>(b.t[2], (g - g2) * TERM_BLOCK + threadIdx.x, x, lambdas, 0.0, red_idx, nullptr,
                                          nullptr, du_dl, u, 0, b.slots[2]);
     }
 }
@@ -307,15 +306,15 @@ void launch_atom_forces(const BondedIncidence &inc, const uint64_t *slots, const
     TM_LAUNCH_CHECK();
 }
 
-void launch_bonded_all(const BondedSet &b, const double *x, const double *lambdas, const int *red_idx, uint64_t *du_dx,
-                       uint64_t *du_dl, uint64_t *u, hipStream_t stream) {
+void launch_bonded_all(const BondedSet &b, const double *x, const double *lambdas, const int *red_idx, uint64_t *du_dl,
+                       uint64_t *u, hipStream_t stream) {
     const int g1 = ceil_div(b.t[0].n, TERM_BLOCK);
     const int g2 = g1 + ceil_div(b.t[1].n, TERM_BLOCK);
     const int grid = g2 + ceil_div(b.t[2].n, TERM_BLOCK);
     if (grid == 0) {
         return;
     }
-    k_bonded_all<<<grid, TERM_BLOCK, 0, stream>>>(b, g1, g2, x, lambdas, red_idx, du_dx, du_dl, u);
+    k_bonded_all<<<grid, TERM_BLOCK, 0, stream>>>(b, g1, g2, x, lambdas, red_idx, du_dl, u);
     TM_LAUNCH_CHECK();
 }
 

@@ -870,7 +870,7 @@ struct Engine::Impl {
                 b.t[k] = {bt_n[k], bt_idx[k].ptr, bt_params[k].ptr, bt_mult[k].ptr, bt_offset[k].ptr, bt_sys[k].ptr};
                 b.slots[k] = ddx ? bt_slots.ptr + static_cast<size_t>(bt_slot0[k]) * 3 : nullptr;
             }
-            launch_bonded_all(b, xp, lamp, red_idx.ptr, nullptr, ddl, uu, st);
+            launch_bonded_all(b, xp, lamp, red_idx.ptr, ddl, uu, st);
         }
         if (ddx) {
             auto sums = [](bool has, const NbState &n) {

@@ -11,8 +11,9 @@
 // 64-bit fixed point per pair and summed exactly (LDS u64 atomics per atom,
 // registers for u and du/dl). Column atoms leave through 64-bit global
 // atomics at the end of each tile, row atoms at the end of a run of tiles of
-// the same row block, u and du/dl with one wave-reduced atomic per system
-// and wave. Integer sums do not depend on the order, so the outputs are
+// the same row block, both to words in sorted order that a second launch moves
+// to the atoms (TileOut); u and du/dl leave once per system and wave
+// (add_scalars). Integer sums do not depend on the order, so the outputs are
 // bitwise those of evaluating the pairs one by one.
 //
 // Pair-list kernel (kernels/k_nonbonded_pair_list.cuh:17-216): one thread
@@ -553,12 +554,24 @@ __device__ __forceinline__ void tile_body(
 
 // Adds a wave's u and du/dl of system s to the outputs. Device-scope atomics on
 // one address take ~10 ns each, one after the other, whoever issues them: the
-// 2100 waves of a 6k-atom system kept u and du/dl busy for 21 us. So the waves w0 .. w1 that work on the system add to NB_RED_SLOTS
-// partial sums in lines of their own, and the last wave of each slot moves its
-// sum to the output and clears the slot for the next launch. Up to RED_DIRECT
-// waves the output's queue is shorter than the two more round trips of a slot.
-// Measured: 48 evaluations of u and du/dl at 4.2k atoms 3.52 -> 3.00 ms, all outputs
-// of 6k atoms with interpolated parameters 339 -> 308 us a call.
+// 2100 waves of a 6k-atom system kept u and du/dl busy for 21 us. So the waves
+// w0 .. w1 that work on the system add to NB_RED_SLOTS partial sums in lines of
+// their own, and the last wave of each slot moves its sum to the output and clears
+// the slot for the next launch. Up to RED_DIRECT waves the output's queue is
+// shorter than the two more round trips of a slot. Measured: 48 evaluations of u
+// and du/dl at 4.2k atoms 3.52 -> 3.00 ms, all outputs of 6k atoms with interpolated
+// parameters 339 -> 308 us a call.
+//
+// The order of a wave's sums and its count. The atomics are relaxed, which in the
+// language's memory model leaves them unordered; what orders them is this
+// hardware. An agent-scope atomic that returns a value returns it from the place
+// where all agent-scope atomics on that line meet (a slot is one 128-byte line), so
+// a sum whose old value has come back is there, and the count is issued after that
+// (it depends on the value). Whoever reads the slot's last count therefore finds
+// every sum with an atomic of its own. A release on the count and an acquire by the
+// last wave say the same in the language, but the release writes the whole L2 back,
+// once a wave: 48 evaluations 2.91 -> 3.71 ms, 30 steps of one 6k system 3.52 -> 4.60
+// ms, u and du/dl at 1k atoms 111 -> 155 us a call.
 constexpr int RED_DIRECT = 256;
 
 template <bool U, bool DL>
@@ -606,7 +619,8 @@ __device__ __forceinline__ void add_scalars(NbRedSlot *slots, const int w, const
 // its row and column atoms and writes both again. Kernel with k_add_sorted, us,
 // whole / halves / quarters / eighths: 153 tiles (1k atoms) 31 / - / - / 13, 801 tiles
 // - / 28 / 22 / 29, 2145 tiles (6k atoms) 48 / 37 / 40 / 56, 4056 tiles 57 / 51 / 62,
-// 8556 tiles 91 / 86, 11304 tiles (35k atoms) 107 whole.
+// 8556 tiles 91 / 86, 11304 tiles (35k atoms) 107 whole. The lines are tile counts for
+// 256 CUs of 16 waves; results do not depend on them.
 __device__ __forceinline__ int tile_split(int tiles) {
     return tiles <= 576 ? 3 : tiles <= 1152 ? 2 : tiles <= 9216 ? 1 : 0;
 }
