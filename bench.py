@@ -43,17 +43,19 @@ PEAK_FP64_TFLOPS = 78.6  # MI355X published FP64 vector peak
 FLOP_PAIR_BASE = 56
 FLOP_PAIR_LJ = 25
 FLOP_PAIR_ALCH = 3
-# The same count for this build's FP64 pair code (nb_pair.h, with its Newton
-# steps and the exp remainder): 71 per pair, + 13 for Lennard-Jones. Reported
-# beside the algorithmic figure, not used for the roofline.
-IMPL_FLOP_PAIR_BASE = 71
-IMPL_FLOP_PAIR_LJ = 13
-# HBM bytes per launch of the du_dx tile kernel on this workload: FETCH_SIZE x 2.0
-# + WRITE_SIZE x 1.0 (factors from a 256 MiB device copy), measured with
+# The same count for this build's FP64 pair code (nb_pair.h and eval_items, with
+# its Newton steps and the exp remainder, in one frame, so without a minimum image):
+# 59 per pair, + 12 for Lennard-Jones. Reported beside the algorithmic figure, not
+# used for the roofline.
+IMPL_FLOP_PAIR_BASE = 59
+IMPL_FLOP_PAIR_LJ = 12
+# HBM bytes of one du_dx force evaluation on this workload, the tile kernel and the
+# move of its sums to the atoms (k_add_sorted; avg_launch_ms holds both): FETCH_SIZE x
+# 2.0 + WRITE_SIZE x 1.0 (factors from a 256 MiB device copy), measured with
 # rocprofv3 --pmc on MI355X (summarised under profiles/ with the commands; the
 # counter program profiles the boxes as built after FIRE, 0.1% fewer tiles than
 # the relaxed state of the kernel trace).
-TILE_TRAFFIC_BYTES = 1.0172e9 + 2.1028e9
+TILE_TRAFFIC_BYTES = (0.8173e9 + 0.7541e9) + (0.0345e9 + 0.1277e9)
 # Serving admits jobs while the resident atoms stay under this: the batched
 # engine's step time is ~0.12 ms + atoms / 3.6e8 atom-steps/s on one MI355X,
 # so 800k resident atoms run at ~95% of the peak rate, and admitting more only

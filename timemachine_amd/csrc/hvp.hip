@@ -297,11 +297,10 @@ __global__ __launch_bounds__(256) void k_pair_list_hvp(const PairListArgs a, con
 }
 
 // All pairs of the tile lists of the last neighborlist build (one or many
-// systems), one wave per tile, in the force kernel's two passes: the screen
-// pairs row lane l with column slot (l + r) mod 64 in round r and compacts the
-// pairs inside the cutoff (FP64 test, as the force kernel) into an LDS queue
-// (ballot / mbcnt); every 64 queued pairs are evaluated one per lane, their
-// fixed-point tangents added to per-atom LDS accumulators of the tile's rows
+// systems), one wave per tile, in two passes: an FP32 screen pairs row lane l with
+// column slot (l + r) mod 64 in round r and compacts the pairs it keeps into an LDS
+// queue (ballot / mbcnt); every 64 queued pairs are evaluated one per lane, with the
+// force kernel's exact FP64 test, their fixed-point tangents added to per-atom LDS accumulators of the tile's rows
 // and columns, which go to global memory once per tile and atom.
 template <int NACC> struct HvpTileLds {
     // [0] rows, [1] columns: position (x, y, z, w), parameters at their FP32
@@ -432,9 +431,10 @@ __global__ __launch_bounds__(64) void k_tiles_hvp(
         const uint32_t islot = L.slot[0][lane];
         // Screen in FP32 with the column values rotating through the wave, on
         // positions relative to the row block's centre from the last build,
-        // imaged once more per pair when the block is too wide for one image
-        // (as the force kernel's pass 1, same margins); eval repeats the exact
-        // FP64 test.
+        // imaged once more per pair when the block is too wide for one image.
+        // FP32 errors stay near 1e-6 relative to the squared cutoff; the margins
+        // are 1e-5, and 1e-4 imaged (coordinates up to L / 2). eval repeats the
+        // exact FP64 test.
         const float4 bc = bb_ctr[Sd.block0 + r];
         const float4 be = bb_ext[Sd.block0 + r];
         const double slack = 0.5 * Sd.padding_d + 1e-4;
