@@ -171,7 +171,10 @@ using PotentialPtr = std::shared_ptr<Potential>;
 // on two streams, so a call's stream first waits for the launches of the call
 // before (an event; nothing waits on the host). A call that is being captured
 // neither waits nor leaves an event: its stream orders it within the graph, and
-// whoever launches the graph orders that with other calls.
+// whoever launches the graph orders that with other calls. The event takes 5 us of a
+// device call that is queued behind others (forces of 2661 atoms 39 -> 44 us, waited
+// for each time 71 -> 73); leaving it out while the stream stays the same would trust
+// a stream's handle, which a later stream may be given again.
 class PotentialCall {
   public:
     PotentialCall(Potential &p, hipStream_t stream, bool host);
